@@ -19,7 +19,7 @@ SOURCES = ["fr_stage64_3d.hip", "fr_stage32_3d.hip", "fr_stage_dbg.hip", "fr_adj
            "fr_batch.hip", "fr_adjoint_v3ad.hip", "fr_api.hip", "fr_host.cpp", "fr_output.cpp", "fr_tri_ops.cpp",
            "fr_tri.hip", "fr_error.hip"]
 HEADERS = ["fr_ctx.hpp", "fr_host.hpp", "fr_kernels.hpp", "fr_layout.hpp", "fr_physics.hpp", "fr_adjoint.hpp",
-           "fr_adjoint_vis.hpp", "fr_dual.hpp", "fr_batch.hpp", "fr_stage_impl.hpp", "fr_tri.hpp"]
+           "fr_adjoint_vis.hpp", "fr_dual.hpp", "fr_batch.hpp", "fr_stage_impl.hpp", "fr_tri.hpp", "fr_viscous.hpp"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -28,6 +28,12 @@ HIPCC_FLAGS = [
     "-fPIC",
     # packed FP32 instructions are disabled for all device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # multiply-adds fused within a source expression only: hipcc's default
+    # also fuses across statements, by the shape of each instance's control
+    # flow, so that two instances of one kernel round differently (a batched
+    # update would not equal a mesh's own; FP32 Rusanov quads differed by up to
+    # 8e-9 after 3 steps).  Costs 0-1 % of the kernels' vector instructions.
+    "-ffp-contract=on",
     "-Wno-unused-result",
 ]
 

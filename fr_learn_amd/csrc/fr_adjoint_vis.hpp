@@ -7,6 +7,7 @@
 
 #include "fr_adjoint.hpp"
 #include "fr_ctx.hpp"
+#include "fr_viscous.hpp"
 
 namespace frimpl {
 
@@ -17,11 +18,21 @@ template <int D, int P, int NF>
 hipError_t vjpViscousLaunchP(fr_ctx *c, const double *Us, const double *lam, double *out, bool bnd) {
   using G = frdev::ElemGeo<D, P>;
   const unsigned nbg = (unsigned)(((c->nE + G::EPB - 1) / G::EPB + 7) / 8 * 8);
-  frdev::GradArgs<double> ga{Us, c->adjTr, c->JG64, c->detJ, c->fgeo64, c->fnbr, c->finfo, c->oned64, c->adjQf,
-                             c->nE, c->ph, /*affine=*/0};
+  frdev::StageArgs<double> ga{};
+  ga.Uin = Us;
+  ga.UfIn = c->adjTr;
+  ga.JG = c->JG64;
+  ga.detJ = c->detJ;
+  ga.fgeo = c->fgeo64;
+  ga.fnbr = c->fnbr;
+  ga.finfo = c->finfo;
+  ga.oned = c->oned64;
+  ga.nEles = c->nE;
+  ga.ph = c->ph;
   const unsigned nbq = (unsigned)(((long)c->nE * G::NFP + 255) / 256);
   if (bnd) {
-    hipLaunchKernelGGL((frdev::k_grad<D, P, NF, double, true>), dim3(nbg), dim3(G::NTH), 0, c->stream, ga);
+    hipLaunchKernelGGL((frdev::k_visc_flux<D, P, NF, double, true, frdev::VISC_GRADIENT>), dim3(nbg), dim3(G::NTH), 0,
+                       c->stream, ga, c->adjQf, (double *)nullptr);
     hipLaunchKernelGGL((frdev::k_vjp_face_vis<D, P, NF, true>), dim3(nbq), dim3(256), 0, c->stream, lam, c->adjTr,
                        c->adjQf, c->adjA, c->fgeo64, c->fnbr, c->finfo, c->oned64, c->ph, c->nE, c->adjUo,
                        c->adjQo, c->adjCj);
@@ -31,7 +42,8 @@ hipError_t vjpViscousLaunchP(fr_ctx *c, const double *Us, const double *lam, dou
     hipLaunchKernelGGL((frdev::k_vjp_ldg<D, P, NF, true>), dim3(c->nE), dim3(G::TPE), 0, c->stream, Us, c->adjB,
                        c->fgeo64, c->fnbr, c->finfo, c->oned64, c->ph, c->nE, out);
   } else {
-    hipLaunchKernelGGL((frdev::k_grad<D, P, NF, double, false>), dim3(nbg), dim3(G::NTH), 0, c->stream, ga);
+    hipLaunchKernelGGL((frdev::k_visc_flux<D, P, NF, double, false, frdev::VISC_GRADIENT>), dim3(nbg), dim3(G::NTH), 0,
+                       c->stream, ga, c->adjQf, (double *)nullptr);
     hipLaunchKernelGGL((frdev::k_vjp_face_vis<D, P, NF, false>), dim3(nbq), dim3(256), 0, c->stream, lam, c->adjTr,
                        c->adjQf, c->adjA, c->fgeo64, c->fnbr, c->finfo, c->oned64, c->ph, c->nE, c->adjUo,
                        c->adjQo, c->adjCj);

@@ -28,10 +28,10 @@ void freeAll(fr_ctx *c) {
   void *bufs[] = {c->U,       c->U0,      c->detJ,    c->JG64,    c->fgeo64, c->ownN,  c->wts,
                   c->oned64,  c->part,    c->U32,     c->JG32,    c->fgeo32, c->oned32, c->Us,
                   c->Uf[0],   c->Uf[1],   c->divF[0], c->divF[1], c->divF[2], c->divF[3], c->fnbr,
-                  c->finfo,   c->dUf,     c->dtG,     c->dtE,     c->adjA,   c->adjTr, c->adjTr2,
+                  c->finfo,   c->Gv,      c->dtG,     c->dtE,     c->adjA,   c->adjTr, c->adjTr2,
                   c->adjLam,  c->adjOut,  c->adjNu,   c->adjW[0], c->adjW[1], c->adjS[0], c->adjS[1],
                   c->adjS[2], c->adjS[3], c->adjQf,   c->adjB,    c->JGc64,  c->detJc, c->fgeoc64,
-                  c->JGc32,   c->fgeoc32, c->adjUo,   c->adjQo,   c->adjCj,   c->Fv,   c->waveSp,
+                  c->JGc32,   c->fgeoc32, c->adjUo,   c->adjQo,   c->adjCj,   c->waveSp,
                   c->dtNum,   c->wsurf,   c->dtPart,  c->geoN64,  c->geoN32,  c->errTab, c->Xd};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
@@ -124,8 +124,8 @@ frdev::StageArgs<T> makeStageArgs(fr_ctx *c, int in, int cur, int mode, int step
   // CFL time stepping: the face fluxes store their wave speeds for the next
   // update's time step (not while the adjoint replays given time steps)
   a.waveSp = (c->dtType != 0 && !c->dtFrozen && !c->tri) ? c->waveSp : nullptr;
-  a.dUf = (const T *)c->dUf;
-  a.Fv = (const T *)c->Fv;
+  a.Gv = (T *)c->Gv;
+  a.divW = (T *)c->divF[step];  // completed in place, also where the update does not keep it
   // Inviscid quads and hexes store no intermediate stage state: a stage that
   // would read Us forms it from the base and the previous stage's residual
   // (the viscous gradient kernel and the triangle kernels read Us itself).
@@ -439,6 +439,7 @@ int stageStates(fr_ctx *c, const double **S) {
     a.UfIn = c->adjTr;
     a.UfOut = c->adjTr2;
     a.divF = nullptr;
+    a.divW = c->adjNu;  // written by vjpStepDev after this
     a.Unext = c->adjS[s + 1];
     a.Uout = nullptr;
     a.Uout32 = nullptr;
@@ -555,10 +556,8 @@ int createImpl(const fr_config *cfg, const fr_mesh *m, int precision, fr_ctx *c)
   HIP_TRY(hipMalloc(&c->Us, nSt * ts));
   if ((rc = dmalloc(&c->dtG, 1))) return rc;
   HIP_TRY(hipMemcpy(c->dtG, &cfg->dt, sizeof(double), hipMemcpyHostToDevice));
-  if (cfg->viscous) {
-    HIP_TRY(hipMalloc(&c->dUf, (size_t)nE * D * c->NF * NFP * ts));
-    HIP_TRY(hipMalloc(&c->Fv, (size_t)nE * c->NF * NFP * ts));
-  }
+  if (cfg->viscous)
+    HIP_TRY(hipMalloc(&c->Gv, (size_t)nE * c->NF * NFP * ts));
   HIP_TRY(hipMemset(c->Us, 0, nSt * ts));
   for (int s = 0; s < c->nRK; s++) {
     HIP_TRY(hipMalloc(&c->divF[s], nSt * ts));
@@ -987,13 +986,14 @@ int fr_get_array(fr_ctx *c, int which, double *out) {
   if (which >= 5 && !c->cfg.viscous) return fail(FR_EINVAL, "fr_get_array: the gradient exists on the viscous path only");
   const int D = c->D, NF = c->NF, NS = c->NS, NFP = c->NFP, nE = c->nE;
   const size_t nSp = (size_t)nE * D * NF * NS, nFp = (size_t)nE * NF * NFP;
-  double *dF = nullptr, *dFn = nullptr, *dJ = nullptr, *dUs = nullptr;
+  double *dF = nullptr, *dFn = nullptr, *dJ = nullptr, *dUs = nullptr, *dUf = nullptr;
   auto release = [&]() {
-    for (double *p : {dF, dFn, dJ, dUs})
+    for (double *p : {dF, dFn, dJ, dUs, dUf})
       if (p) (void)hipFree(p);
   };
   if (hipMalloc(&dF, nSp * 8) != hipSuccess || hipMalloc(&dFn, nFp * 8) != hipSuccess ||
-      hipMalloc(&dJ, nFp * 8) != hipSuccess || (c->cfg.viscous && hipMalloc(&dUs, nSp * 8) != hipSuccess)) {
+      hipMalloc(&dJ, nFp * 8) != hipSuccess ||
+      (c->cfg.viscous && (hipMalloc(&dUs, nSp * 8) != hipSuccess || hipMalloc(&dUf, nFp * D * 8) != hipSuccess))) {
     release();
     return fail(FR_EHIP, "fr_get_array: device allocation failed");
   }
@@ -1005,12 +1005,12 @@ int fr_get_array(fr_ctx *c, int which, double *out) {
     a.dbgF = dF;
     a.dbgFn = dFn;
     a.dbgJ = dJ;
-    rc = launchStageDbg(c, a, dUs);
+    rc = launchStageDbg(c, a, dUf, dUs);
   }
   hipError_t err = hipStreamSynchronize(c->stream);
   std::vector<double> h;
   if (!rc && err == hipSuccess) {
-    const double *src = which == 2 ? dF : which == 3 ? dFn : which == 4 ? dJ : which == 5 ? dUs : (const double *)c->dUf;
+    const double *src = which == 2 ? dF : which == 3 ? dFn : which == 4 ? dJ : which == 5 ? dUs : dUf;
     h.resize(which == 6 ? (size_t)nE * D * NF * NFP : (which == 2 || which == 5) ? nSp : nFp);
     err = hipMemcpy(h.data(), src, h.size() * 8, hipMemcpyDeviceToHost);
   }

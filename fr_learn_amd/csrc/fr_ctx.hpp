@@ -93,8 +93,7 @@ struct fr_ctx {
   int keepFinal = 1;                  // the final RK stage stores divF_spts[nRK-1] (fr_keep_final_residual)
   bool finalDropped = false;          // divF[nRK-1] is stale: the last update did not store it
   void *divF[4] = {nullptr, nullptr, nullptr, nullptr};
-  void *dUf = nullptr;                // viscous: gradient traces [ele][dim][field][fpt]
-  void *Fv = nullptr;                 // viscous: common viscous normal flux [ele][field][fpt]
+  void *Gv = nullptr;                 // viscous: each side's share of the common flux [ele][field][fpt]
   double *dtG = nullptr;              // the global time step (one value)
   double *dtE = nullptr;              // per-element time steps (local time stepping)
   int dtType = 0;                     // 0 fixed dt, 1 global CFL dt, 2 local CFL dt
@@ -224,8 +223,9 @@ template <typename T>
 int launchStageArgs(fr_ctx *c, const frdev::StageArgs<T> &a, int mode);
 // The residual evaluation of arguments `a` (mode 0, FP64, quads and hexes)
 // with its debug outputs (a.dbgF, a.dbgFn, a.dbgJ; on the viscous path the
-// gradient at the spts into dUs), fr_stage_dbg.hip.
-int launchStageDbg(fr_ctx *c, const frdev::StageArgs<double> &a, double *dUs);
+// gradient traces into dUf and the gradient at the spts into dUs),
+// fr_stage_dbg.hip.
+int launchStageDbg(fr_ctx *c, const frdev::StageArgs<double> &a, double *dUf, double *dUs);
 // (d divF / dU)^T lam at the state Us, device arrays (fr_adjoint.hip).
 int vjpResidualDev(fr_ctx *c, const double *Us, const double *lam, double *out);
 // triangle kernels (fr_tri.hip)

@@ -10,7 +10,7 @@
 //                                 c == D: this element's own dA
 //   fnbr          [ele][face]     neighbour element (interior faces)
 //   finfo         [ele][face]     packed face record (fr_layout.hpp packFinfo)
-//   dUf           [ele][dim][field][fpt]  gradient traces (viscous only)
+//   Gv            [ele][field][fpt]  a side's share of the common flux (viscous only, fr_viscous.hpp)
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -25,9 +25,6 @@
 #endif
 #ifndef FR_MFMA
 #define FR_MFMA 1  // hex P3 inviscid stages: the line contractions of F~ on the matrix cores
-#endif
-#ifndef FR_FOLD
-#define FR_FOLD 1  // stage kernels: the jump correction folded into the derivative
 #endif
 #ifndef FR_INBLOCK
 #define FR_INBLOCK 1  // neighbours in the same workgroup: traces extrapolated from their LDS state (VALU variants)
@@ -242,8 +239,8 @@ struct StageArgs {
   const T *dprev0, *dprev1, *dprev2;
   const T *rprev;  // previous stage's residual, or null (stage state in Uin)
   double rkPrev;   // its coefficient in the stage state
-  const T *__restrict__ dUf;  // viscous: gradient traces [ele][dim][field][fpt]
-  const T *__restrict__ Fv;   // viscous: common viscous normal flux [ele][field][fpt] (k_vflux)
+  T *__restrict__ Gv;         // viscous: each side's share of the common normal flux [ele][field][fpt] (k_visc_flux)
+  T *divW;                    // viscous: divergence of the point fluxes, before the correction [ele][field][spt]
   const double *dtE;          // time step: dtE[ele * dtStride] (stride 0: one global dt)
   int dtStride;
   double *waveSp;             // CFL wave speeds [ele][fpt] written at left / boundary points, or null
@@ -299,13 +296,13 @@ __device__ __forceinline__ int faceAxis(int f) {
 template <int D, int NF, typename T>
 __device__ __forceinline__ void ldgJump(const Phys &ph, bool bnd, bool right, const T *uo, const T *un, const T *n,
                                         T *dUc) {
+  // UC = (uL + uR) / 2 - pen (uL - uR) inside, (uL + ghost) / 2 at boundaries;
+  // less the own trace that is (un - uo) times 1/2, plus pen on the left side
+  // and minus pen on the right
   const T pen = bnd ? (T)0 : ldgPenalty<D, T>(ph, n);
+  const T w = (T)0.5 + (right ? -pen : pen);
 #pragma unroll
-  for (int k = 0; k < NF; k++) {
-    const T UL = right ? un[k] : uo[k], UR = right ? uo[k] : un[k];
-    const T UC = bnd ? (T)0.5 * (UL + UR) : (T)0.5 * (UL + UR) - pen * (UL - UR);
-    dUc[k] = UC - uo[k];
-  }
+  for (int k = 0; k < NF; k++) dUc[k] = w * (un[k] - uo[k]);
 }
 
 // Hex P3 line operations on the matrix cores.  One element is one wavefront,
@@ -441,18 +438,40 @@ __device__ __forceinline__ double lanePull(int addr, double v) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-// Phase (2) on the matrix cores: per reference axis d the contravariant
-// flux F~_d = sum_d2 JGinv(d,d2) F_d2, its derivative along d added to div,
-// and its values at the two faces normal to d, stored negated as the start
-// of the jump (the left face's outward flux is -F~_d): sJ at the round-0
-// and round-1 flux points of the lane.  FD: the folded derivative
-// (OneD::DMF) alone, no face values (the jump is the common flux alone).
-template <int NF, typename T, bool FD = false, typename SM>
+// The divergence of a hex P3 element on the matrix cores: per reference axis d
+// the contravariant flux F~_d = sum_d2 JGinv(d,d2) F_d2 and its folded
+// derivative (OneD::DMF) along d, summed over the axes.  All lanes take part.
+template <int NF, typename T>
+__device__ __forceinline__ void mfmaDivergence(const T *s1, const int t, const T *pJ, const T (&F)[3][NF],
+                                               T (&div)[NF]) {
+  using V = MfmaVec<T>;
+  const MfmaLane<T> L(s1, t, true);
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+#pragma unroll
+    for (int k = 0; k < NF; k++) {
+      T ft = (T)0;
+#pragma unroll
+      for (int d2 = 0; d2 < 3; d2++) ft += pJ[d * 3 + d2] * F[d2][k];
+      const T b = d < 2 ? lanePull(d == 0 ? L.bx : L.by, ft) : ft;
+      const T der = V::der(L.aD, d == 0 ? L.aEx : L.aEzy, b);
+      const T dv = d < 2 ? lanePull(d == 0 ? L.ix : L.iy, der) : der;
+      div[k] = d == 0 ? dv : dv + div[k];
+    }
+  }
+}
+
+// Phase (2) of the debug instance on the matrix cores: per reference axis d the
+// contravariant flux F~_d (to dbgF), its derivative along d added to div, and
+// its values at the two faces normal to d, stored negated as the start of the
+// jump (the left face's outward flux is -F~_d): sJ at the round-0 and round-1
+// flux points of the lane.
+template <int NF, typename T, typename SM>
 __device__ __forceinline__ void mfmaAxes(SM &sm, const int slot, const int t, const T *pJ, const T (&F)[3][NF],
                                          T (&div)[NF], T *dbgF) {
   using V = MfmaVec<T>;
   auto &sJ = sm.sJ;
-  const MfmaLane<T> L(sm.s1, t, FD);
+  const MfmaLane<T> L(sm.s1, t);
   T e0[NF], e1[NF];
 #pragma unroll
   for (int k = 0; k < NF; k++) e0[k] = e1[k] = (T)0;
@@ -463,23 +482,20 @@ __device__ __forceinline__ void mfmaAxes(SM &sm, const int slot, const int t, co
       T ft = (T)0;
 #pragma unroll
       for (int d2 = 0; d2 < 3; d2++) ft += pJ[d * 3 + d2] * F[d2][k];
-      if (dbgF) dbgF[(d * NF + k) * 64 + t] = ft;
+      dbgF[(d * NF + k) * 64 + t] = ft;
       const T b = d < 2 ? lanePull(d == 0 ? L.bx : L.by, ft) : ft;
       T der;
-      if constexpr (FD) der = V::der(L.aD, d == 0 ? L.aEx : L.aEzy, b);
-      else V::axis(L.aD, d == 0 ? L.aEx : L.aEzy, b, d == 1 ? e1[k] : e0[k], der);
+      V::axis(L.aD, d == 0 ? L.aEx : L.aEzy, b, d == 1 ? e1[k] : e0[k], der);
       const T dv = d < 2 ? lanePull(d == 0 ? L.ix : L.iy, der) : der;
       div[k] = d == 0 ? dv : dv + div[k];
     }
   }
-  if constexpr (!FD) {
-    const T sg = ((t >> 4) & 1) ? (T)-1 : (T)1;
-    const int q0 = mfmaFpt(t, 0), q1 = mfmaFpt(t, 1);
+  const T sg = ((t >> 4) & 1) ? (T)-1 : (T)1;
+  const int q0 = mfmaFpt(t, 0), q1 = mfmaFpt(t, 1);
 #pragma unroll
-    for (int k = 0; k < NF; k++) {
-      sJ[slot][k][q0] = sg * e0[k];
-      if (t < 32) sJ[slot][k][q1] = sg * e1[k];
-    }
+  for (int k = 0; k < NF; k++) {
+    sJ[slot][k][q0] = sg * e0[k];
+    if (t < 32) sJ[slot][k][q1] = sg * e1[k];
   }
   elementSync<64>();
 }
@@ -512,6 +528,25 @@ __device__ __forceinline__ void mfmaFaceRoundReg(const T *s1, const int t, const
                   : V::ext(L.aEzy, lanePull(L.by, own[k]), (T)0);
 }
 
+// The physical gradient JGinv^T gr / detJ of a reference-space gradient gr at
+// one point, J = JGinv(dimRef, dimPhys).
+template <int D, int NF, typename T>
+__device__ __forceinline__ void physicalGradient(const T gr[D][NF], const T *J, T detJ, T g[D][NF]) {
+  const T invDet = recip(detJ);
+#pragma unroll
+  for (int d1 = 0; d1 < D; d1++) {
+    T Jd[D];
+#pragma unroll
+    for (int d = 0; d < D; d++) Jd[d] = J[d * D + d1] * invDet;
+#pragma unroll
+    for (int k = 0; k < NF; k++) {
+      T acc = gr[0][k] * Jd[0] + gr[1][k] * Jd[1];
+      if constexpr (D == 3) acc = acc + gr[2][k] * Jd[2];
+      g[d1][k] = acc;
+    }
+  }
+}
+
 // correctedGradient (below) for hex P3 with the reference-space derivative on
 // the matrix cores: the state S in LDS (fields RS apart, padded rows when
 // PADV) and the lane's own values own[], the jumps sCe [NF][NFP] at flux
@@ -526,6 +561,9 @@ __device__ __forceinline__ void mfmaGradient(const T *s1, const T *S, const T (&
   const MfmaLane<T> L(s1, t);
   int cq[NFACE], cside[NFACE], cax[NFACE];
   corrEntries<3, 3>(t, cq, cside, cax);
+  T cw[NFACE];  // lift weights, read once for all fields
+#pragma unroll
+  for (int f = 0; f < NFACE; f++) cw[f] = cside[f] ? s1[O::GR + cax[f]] : -s1[O::GL + cax[f]];
   T gr[3][NF];
 #pragma unroll
   for (int d = 0; d < 3; d++) {
@@ -537,20 +575,11 @@ __device__ __forceinline__ void mfmaGradient(const T *s1, const T *S, const T (&
       T corr = (T)0;
 #pragma unroll
       for (int f = 0; f < NFACE; f++)
-        if (faceAxis<3>(f) == d)
-          corr += (s1[(cside[f] ? O::GR : O::GL) + cax[f]] * (cside[f] ? (T)1 : (T)-1)) * sCe[k * NFP + cq[f]];
+        if (faceAxis<3>(f) == d) corr += cw[f] * sCe[k * NFP + cq[f]];
       gr[d][k] = corr + dv;
     }
   }
-  const T invDet = (T)1. / detJ;
-#pragma unroll
-  for (int d1 = 0; d1 < 3; d1++)
-#pragma unroll
-    for (int k = 0; k < NF; k++) {
-      T acc = gr[0][k] * J[0 * 3 + d1] + gr[1][k] * J[1 * 3 + d1];
-      acc = acc + gr[2][k] * J[2 * 3 + d1];
-      g[d1][k] = invDet * acc;
-    }
+  physicalGradient<3, NF, T>(gr, J, detJ, g);
 }
 
 // Corrected physical gradient at solution point t (calcGradU_spts,
@@ -569,6 +598,9 @@ __device__ __forceinline__ void correctedGradient(const T *s1, const T *sUe, con
   constexpr int NS = PAD ? G::NSP : G::NS;
   int cq[NFACE], cside[NFACE], cax[NFACE];
   corrEntries<D, P>(t, cq, cside, cax);
+  T cw[NFACE];  // lift weights, read once for all fields
+#pragma unroll
+  for (int f = 0; f < NFACE; f++) cw[f] = cside[f] ? s1[O::GR + cax[f]] : -s1[O::GL + cax[f]];
   T gr[D][NF];
 #pragma unroll
   for (int d = 0; d < D; d++) {
@@ -584,262 +616,11 @@ __device__ __forceinline__ void correctedGradient(const T *s1, const T *sUe, con
       T corr = (T)0;
 #pragma unroll
       for (int f = 0; f < NFACE; f++)
-        if (faceAxis<D>(f) == d)
-          corr += (s1[(cside[f] ? O::GR : O::GL) + cax[f]] * (cside[f] ? (T)1 : (T)-1)) * sCe[k * NFP + cq[f]];
+        if (faceAxis<D>(f) == d) corr += cw[f] * sCe[k * NFP + cq[f]];
       gr[d][k] = corr + acc;
     }
   }
-  const T invDet = (T)1. / detJ;
-#pragma unroll
-  for (int d1 = 0; d1 < D; d1++)
-#pragma unroll
-    for (int k = 0; k < NF; k++) {
-      T acc = gr[0][k] * J[0 * D + d1] + gr[1][k] * J[1 * D + d1];
-      if constexpr (D == 3) acc = acc + gr[2][k] * J[2 * D + d1];
-      g[d1][k] = invDet * acc;
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Viscous common normal flux at every flux point (face::calcViscousFlux,
-// face.cpp:177-287), one thread per (element, flux point), from the state
-// traces UfIn and the gradient traces dUf: boundaries take
-// boundFace::applyViscousBCs (boundFace.cpp:279-320), advection-diffusion
-// boundaries a zero outside gradient.  Right-side points evaluate it in the
-// left element's frame, as the inviscid flux.  Fv[ele][field][fpt] (before
-// the dA scaling), which the viscous stage kernel adds to its inviscid
-// common flux: one thread per point keeps the stage kernel's registers for
-// the rest of its work.
-// ---------------------------------------------------------------------------
-template <int D, int P, int NF, typename T, bool BND>
-__global__ __launch_bounds__(256) void k_vflux(const T *__restrict__ Uf, const T *__restrict__ dUf,
-                                               const T *__restrict__ fgeo, const int32_t *__restrict__ fnbr,
-                                               const int8_t *__restrict__ finfo, int affine, Phys ph, int nEles,
-                                               T *__restrict__ Fv) {
-  using G = ElemGeo<D, P>;
-  constexpr int NFP = G::NFP, NFPF = G::NFPF, NFACE = G::NFACE;
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)nEles * NFP) return;
-  const size_t e = (size_t)(idx / NFP);
-  const int q = (int)(idx - (long)e * NFP);
-  const GeoAddr<D, P> ga(affine, 0);
-  const int fi = finfo[e * NFACE + q / NFPF];
-  const bool bnd = BND && fi >= FINFO_BOUNDARY;
-  const bool right = !bnd && ((fi >> 5) & 1);
-  T n[D], uo[NF], un[NF], go[D][NF], gn[D][NF], F[NF];
-#pragma unroll
-  for (int c = 0; c < D; c++) n[c] = fgeo[ga.fg(e, c, q)];
-#pragma unroll
-  for (int k = 0; k < NF; k++) {
-    uo[k] = Uf[(e * NF + k) * NFP + q];
-    F[k] = (T)0;
-  }
-  const T *Go = dUf + e * D * NF * NFP + q;
-#pragma unroll
-  for (int d = 0; d < D; d++)
-#pragma unroll
-    for (int k = 0; k < NF; k++) go[d][k] = Go[(d * NF + k) * NFP];
-  int vb = 0;
-  if (bnd) {
-    const int bc = fi - FINFO_BOUNDARY;
-    vb = (bc == 10) ? 2 : 1;
-    boundaryState<D, NF, T>(ph, bc, uo, n, un);
-    if constexpr (NF > 1) {
-      boundaryGradient<D, NF, T>(ph, bc, uo, un, go, gn);
-    } else {
-#pragma unroll
-      for (int d = 0; d < D; d++) gn[d][0] = (T)0;
-    }
-  } else {
-    const size_t en = (size_t)fnbr[e * NFACE + q / NFPF];
-    const int qn = neighbourFpt<D, P>(q, fi);
-#pragma unroll
-    for (int k = 0; k < NF; k++) un[k] = Uf[(en * NF + k) * NFP + qn];
-    const T *Gn = dUf + en * D * NF * NFP + qn;
-#pragma unroll
-    for (int d = 0; d < D; d++)
-#pragma unroll
-      for (int k = 0; k < NF; k++) gn[d][k] = Gn[(d * NF + k) * NFP];
-  }
-  if (right) ldgViscousFlux<D, NF, T>(ph, 0, un, uo, gn, go, n, F);
-  else ldgViscousFlux<D, NF, T>(ph, vb, uo, un, go, gn, n, F);
-#pragma unroll
-  for (int k = 0; k < NF; k++) Fv[(e * NF + k) * NFP + q] = F[k];
-}
-
-// ---------------------------------------------------------------------------
-// Gradient traces for the viscous path: LDG common solution at every flux
-// point, corrected physical gradient at the solution points, and its
-// extrapolation to the flux points (extrapolateGradU, solver.cpp:881-895),
-// written to dUf[ele][dim][field][fpt] for the neighbours' viscous face flux.
-// ---------------------------------------------------------------------------
-template <typename T>
-struct GradArgs {
-  const T *__restrict__ Uin;
-  const T *__restrict__ UfIn;
-  const T *__restrict__ JG;
-  const double *__restrict__ detJ;
-  const T *__restrict__ fgeo;
-  const int32_t *__restrict__ fnbr;
-  const int8_t *__restrict__ finfo;
-  const T *__restrict__ oned;
-  T *__restrict__ dUf;
-  int nEles;
-  Phys ph;
-  int affine;  // geometry layout (GeoAddr)
-  T *dUs;      // debug output (null in production launches): the gradient at the spts [ele][dim][field][spt]
-};
-
-template <int D, int P, int NF, typename T, bool BND>
-__global__ __launch_bounds__((ElemGeo<D, P>::NTH)) void k_grad(GradArgs<T> a) {
-  using G = ElemGeo<D, P>;
-  using O = OneD<P>;
-  constexpr int NS = G::NS, NFP = G::NFP, NFPF = G::NFPF, P1 = G::P1, TPE = G::TPE, EPB = G::EPB;
-  constexpr int NFACE = G::NFACE, NQ = (NFP + TPE - 1) / TPE;
-  __shared__ T sU[EPB][NF][NS];
-  __shared__ T sC[EPB][NF][NFP];
-  // the gradient at the solution points for its traces (the matrix-core
-  // variant takes them from the lanes' registers instead)
-  constexpr bool MG0 = FR_MFMA && D == 3 && P == 3 && sizeof(T) == 8;
-  __shared__ T sG[MG0 ? 1 : EPB][D][NF][MG0 ? 1 : NS];
-  __shared__ T s1[O::SIZE];
-  const int b = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  const int slot = threadIdx.x / TPE, t = threadIdx.x - slot * TPE;
-  const int e = b * EPB + slot;
-  const bool act = e < a.nEles;
-  // hex P3 FP64: the state's face values, the gradient's derivative and the
-  // gradient traces on the matrix cores (lane t handles flux point
-  // mfmaFpt(t, r) in round r)
-  constexpr bool MG = FR_MFMA && D == 3 && P == 3 && sizeof(T) == 8;
-  const bool hasS = act && t < NS;
-  for (int i = threadIdx.x; i < O::SIZE; i += blockDim.x) s1[i] = a.oned[i];
-  if (act) {
-    const T *Ue = a.Uin + (size_t)e * NF * NS;
-    for (int i = t; i < NF * NS; i += TPE) (&sU[slot][0][0])[i] = Ue[i];
-  }
-  T pJ[D * D];
-  T pdet = (T)1;
-  const GeoAddr<D, P> ga(a.affine, t);
-  if (hasS) {
-#pragma unroll
-    for (int c = 0; c < D * D; c++) pJ[c] = a.JG[ga.jg(e, c)];
-    pdet = (T)a.detJ[ga.det(e)];
-  }
-  __syncthreads();
-  // LDG jump at every flux point
-#pragma unroll
-  for (int r = 0; r < NQ; r++) {
-    const int q = MG ? mfmaFpt(t, r) : t + r * TPE;
-    T uo[NF];
-    if constexpr (MG) {
-      if (act) {
-        T own[NF];
-#pragma unroll
-        for (int k = 0; k < NF; k++) own[k] = sU[slot][k][t];
-        mfmaFaceRound<NF, NS, T, false>(s1, &sU[slot][0][0], t, own, r, uo);
-      }
-    }
-    if (act && q < NFP) {
-      int base, stride, side, dn;
-      fptLine<D, P>(q, base, stride, side, dn);
-      const T *l1 = s1 + (side ? O::LR : O::LL);
-      T un[NF], n[D], dUc[NF];
-      if constexpr (!MG) {
-#pragma unroll
-        for (int k = 0; k < NF; k++) {
-          T acc = (T)0;
-#pragma unroll
-          for (int m = 0; m < P1; m++) acc += l1[m] * sU[slot][k][base + m * stride];
-          uo[k] = acc;
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < D; c++) n[c] = a.fgeo[ga.fg(e, c, q)];
-      const int fi = a.finfo[(size_t)e * NFACE + q / NFPF];
-      const bool bnd = BND && fi >= FINFO_BOUNDARY;
-      if (bnd) {
-        boundaryState<D, NF, T>(a.ph, fi - FINFO_BOUNDARY, uo, n, un);
-      } else {
-        const T *Ur = a.UfIn + (size_t)a.fnbr[(size_t)e * NFACE + q / NFPF] * NF * NFP + neighbourFpt<D, P>(q, fi);
-#pragma unroll
-        for (int k = 0; k < NF; k++) un[k] = Ur[k * NFP];
-      }
-      ldgJump<D, NF, T>(a.ph, bnd, !bnd && ((fi >> 5) & 1), uo, un, n, dUc);
-#pragma unroll
-      for (int k = 0; k < NF; k++) sC[slot][k][q] = dUc[k];
-    }
-  }
-  elementSync<TPE>();
-  T g[D][NF];
-  if (MG && act) {
-    if constexpr (MG) {
-      T own[NF];
-#pragma unroll
-      for (int k = 0; k < NF; k++) own[k] = sU[slot][k][t];
-      mfmaGradient<NF, NS, T, false>(s1, &sU[slot][0][0], own, &sC[slot][0][0], t, pJ, pdet, g);
-      if (a.dUs)
-#pragma unroll
-        for (int d = 0; d < D; d++)
-#pragma unroll
-          for (int k = 0; k < NF; k++) a.dUs[(((size_t)e * D + d) * NF + k) * NS + t] = g[d][k];
-    }
-  } else if (hasS) {
-    int si, sj, sk;
-    if (D == 3) {
-      sk = t / (P1 * P1);
-      sj = (t - P1 * P1 * sk) / P1;
-      si = t - P1 * sj - P1 * P1 * sk;
-    } else {
-      si = t % P1;
-      sj = t / P1;
-      sk = 0;
-    }
-    correctedGradient<D, P, NF, T>(s1, &sU[slot][0][0], &sC[slot][0][0], t, si, sj, sk, pJ, pdet, g);
-#pragma unroll
-    for (int d = 0; d < D; d++)
-#pragma unroll
-      for (int k = 0; k < NF; k++) sG[slot][d][k][t] = g[d][k];
-    if (a.dUs)
-#pragma unroll
-      for (int d = 0; d < D; d++)
-#pragma unroll
-        for (int k = 0; k < NF; k++) a.dUs[(((size_t)e * D + d) * NF + k) * NS + t] = g[d][k];
-  }
-  elementSync<TPE>();
-  if (MG && act) {
-    if constexpr (MG) {
-      T *Ge = a.dUf + (size_t)e * D * NF * NFP;
-#pragma unroll
-      for (int r = 0; r < NQ; r++) {
-        const int q = mfmaFpt(t, r);
-#pragma unroll
-        for (int d = 0; d < D; d++) {
-          T v[NF];
-          mfmaFaceRoundReg<NF, T>(s1, t, g[d], r, v);
-          if (q < NFP)
-#pragma unroll
-            for (int k = 0; k < NF; k++) Ge[(d * NF + k) * NFP + q] = v[k];
-        }
-      }
-    }
-  } else if (act) {
-    T *Ge = a.dUf + (size_t)e * D * NF * NFP;
-#pragma unroll 1
-    for (int q = t; q < NFP; q += TPE) {
-      int base, stride, side, dn;
-      fptLine<D, P>(q, base, stride, side, dn);
-      const T *l1 = s1 + (side ? O::LR : O::LL);
-#pragma unroll
-      for (int d = 0; d < D; d++)
-#pragma unroll
-        for (int k = 0; k < NF; k++) {
-          T acc = (T)0;
-#pragma unroll
-          for (int m = 0; m < P1; m++) acc += l1[m] * sG[slot][d][k][base + m * stride];
-          Ge[(d * NF + k) * NFP + q] = acc;
-        }
-    }
-  }
+  physicalGradient<D, NF, T>(gr, J, detJ, g);
 }
 
 // LDS of one stage-kernel workgroup (tile layout L).
@@ -852,11 +633,117 @@ struct StageSmem {
   T s1[OneD<P>::SIZE];        // 1D factor table
 };
 
+// The end of a stage, phases (4) and (5) of stageBody: the correction of the
+// jumps sJe [NF][NFP] (correctDivFlux, solver.cpp:789-806) added to the
+// divergence div, the stage update from the base pb (final stages: with the
+// earlier residuals' terms already subtracted), and the face traces of the
+// updated state, staged in sSe [NF][NSP].  face(r) is false for the rounds
+// whose flux point needs no trace in HBM.
+template <int D, int P, int NF, typename T, bool FIN, bool DEF, int L, typename Face>
+__device__ __forceinline__ void stageUpdate(const StageArgs<T> &a, const T *s1, const T *sJe, T *sSe, const int e,
+                                            const int t, const bool act, const T *div, const double *pb,
+                                            const double pdet, const double pdt, Face face) {
+  using G = ElemGeo<D, P, L>;
+  using O = OneD<P>;
+  constexpr int NS = G::NS, NSP = G::NSP, NFP = G::NFP, P1 = G::P1, TPE = G::TPE, NFACE = G::NFACE;
+  constexpr int NQ = (NFP + TPE - 1) / TPE;
+  constexpr bool MF = FR_MFMA && D == 3 && P == 3, MFF = MF && sizeof(T) == 8;
+  // the FP64 base of the final stages is absolute; FP32 stage states hold the
+  // energy less Phys::eOff
+  constexpr bool base64 = FIN;
+  T utv[NF];  // the updated state at this thread's point
+  if (act && t < NS) {
+    int cq[NFACE], cside[NFACE], cax[NFACE];
+    corrEntries<D, P>(t, cq, cside, cax);
+    T cw[NFACE];  // correction weights, read once for all fields
+#pragma unroll
+    for (int f = 0; f < NFACE; f++) cw[f] = s1[(cside[f] ? O::GR : O::GL) + cax[f]];
+    const size_t eo = (size_t)e * NF * NS;
+#pragma unroll
+    for (int k = 0; k < NF; k++) {
+      T corr = (T)0;
+#pragma unroll
+      for (int f = 0; f < NFACE; f++) corr += cw[f] * sJe[k * NFP + cq[f]];
+      const T dv = corr + div[k];
+      const size_t gi = eo + (size_t)k * NS + t;
+      if (a.divF) __builtin_nontemporal_store(dv, a.divF + gi);
+      if (!FIN && a.mode == 0) continue;
+      // stage terms RK * divF / detJ * dt, with dt / detJ formed once per point
+      const double dtJ = pdt / pdet;
+      double u = pb[k];
+      // DEF: the base state read again here instead of kept in registers
+      if constexpr (DEF) u = (double)a.UbaseT[gi];
+      if (FIN && a.mode == 2) {
+        // earlier residuals: already subtracted from pb
+        const double cl = (a.nprev == 0) ? a.c0 : (a.nprev == 1) ? a.c1 : (a.nprev == 2) ? a.c2 : a.c3;
+        u -= cl * (double)dv * dtJ;
+      } else {
+        u = u - a.rk * (double)dv * dtJ;
+      }
+      // the updated state in the residual precision, for the traces
+      double ut = u;
+      if constexpr (hasEnergyOffset<T>())
+        if (k == NF - 1 && base64) ut = u - a.ph.eOff;
+      if constexpr (!FIN) {
+        if (a.Unext) __builtin_nontemporal_store((T)u, a.Unext + gi);
+      } else {
+        __builtin_nontemporal_store(u, a.Uout + gi);
+        if (a.Uout32) __builtin_nontemporal_store((float)ut, a.Uout32 + gi);
+      }
+      sSe[k * NSP + padIdx<P>(t)] = (T)ut;
+      utv[k] = (T)ut;
+    }
+  }
+  if (!FIN && a.mode == 0) return;
+  elementSync<TPE>();
+  if (!act) return;
+  T *Fe = a.UfOut + (size_t)e * NF * NFP;
+#pragma unroll
+  for (int r = 0; r < NQ; r++) {
+    const int q = MF ? mfmaFpt(t, r) : t + r * TPE;
+    T tv[NF];
+    if constexpr (MFF) mfmaFaceRound<NF, NSP, T>(s1, sSe, t, utv, r, tv);
+    if (q >= NFP || !face(r)) continue;
+    if constexpr (MFF) {
+#pragma unroll
+      for (int k = 0; k < NF; k++) __builtin_nontemporal_store(tv[k], Fe + k * NFP + q);
+      continue;
+    }
+    int base, stride, side, dn;
+    fptLine<D, P>(q, base, stride, side, dn);
+    const int lb = padIdx<P>(base), ls = padStride<P>(stride);
+    const T *l1 = s1 + (side ? O::LR : O::LL);
+#pragma unroll
+    for (int k = 0; k < NF; k++) {
+      T acc = (T)0;
+#pragma unroll
+      for (int m = 0; m < P1; m++) acc += l1[m] * sSe[k * NSP + lb + m * ls];
+      __builtin_nontemporal_store(acc, Fe + k * NFP + q);
+    }
+  }
+}
+
+// The earlier residuals' terms of the final update (mode 2), subtracted from
+// the base in stage order as the timeStepB passes do.
+template <int NF, typename T>
+__device__ __forceinline__ void subtractEarlier(const StageArgs<T> &a, const T (&pd)[3][NF], const double dtJ,
+                                                double *pb) {
+#pragma unroll
+  for (int k = 0; k < NF; k++) {
+    double u = pb[k];
+    if (a.nprev > 0) u -= a.c0 * (double)pd[0][k] * dtJ;
+    if (a.nprev > 1) u -= a.c1 * (double)pd[1][k] * dtJ;
+    if (a.nprev > 2) u -= a.c2 * (double)pd[2][k] * dtJ;
+    pb[k] = u;
+  }
+}
+
 // BND = false is the variant for meshes without boundary faces (no ghost
-// states, which keeps its register allocation small).  VIS adds the viscous
-// terms (LDG): the corrected gradient at the solution points is recomputed
-// here from the state and the neighbours' traces exactly as k_grad forms it,
-// and the viscous common flux reads the gradient traces k_grad wrote.
+// states, which keeps its register allocation small).  VIS (the debug
+// instance only: a production stage of the viscous path is the two kernels of
+// fr_viscous.hpp) adds the viscous terms (LDG): the corrected gradient at the
+// solution points from the state and the neighbours' traces, and the common
+// flux from the shares k_visc_flux wrote.
 // FIN = true is the variant for the final stages (modes 2 and 3): the FP64
 // base state, and in mode 2 the earlier stages' residuals, are prefetched.
 // FIN = false serves modes 0 and 1 with the base in the residual precision.
@@ -884,9 +771,6 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
   auto &sFd = sm.sFd;
   auto &sJ = sm.sJ;
   auto &s1 = sm.s1;
-  // the modes a variant serves: the inviscid FIN variants 2 and 3, the other
-  // inviscid variants 0 and 1 (the launches choose so), the viscous one all
-  constexpr bool M01 = VIS || !FIN, M23 = VIS || FIN;
   // hex P3: the line contractions of (2) on the matrix cores
   constexpr bool MF = FR_MFMA && D == 3 && P == 3;
   // the face values of the state in (3) and (5) too: FP64 only (three FP32
@@ -897,7 +781,7 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
   // common flux alone (the viscous variant's LDG jumps of (0), held in sJ, are
   // read in (1), before (2)'s barriers; the debug instance keeps the jump it
   // reports)
-  constexpr bool FOLD = FR_FOLD && !DBG;
+  constexpr bool FOLD = !DBG;
   const int slot = tid / TPE, t = tid - slot * TPE;
   const int tP = padIdx<P>(t);  // padded LDS index of this thread's solution point
   // flux point of this thread in round r of the face phases: the matrix-core
@@ -981,13 +865,12 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
   const double pdt = a.dtE[ec * a.dtStride];
 #pragma unroll
   for (int k = 0; k < NF; k++)
-    pb[k] = (FIN || (VIS && a.mode >= 2)) ? a.Ubase[(ec * NF + k) * NS + tc]
-                                          : (double)a.UbaseT[(ec * NF + k) * NS + tc];
+    pb[k] = FIN ? a.Ubase[(ec * NF + k) * NS + tc] : (double)a.UbaseT[(ec * NF + k) * NS + tc];
   // earlier stages' residuals for the final update, issued with the state:
   // they are folded into the base before the barrier, which frees their
   // registers for the LDS phases (the latest one is already in ul when rprev
   // is set)
-  T pd[FIN ? 3 : 1][NF];
+  T pd[3][NF];
   if constexpr (FIN) {
     const T *dp[3] = {a.dprev0, a.dprev1, a.dprev2};
 #pragma unroll
@@ -1034,7 +917,7 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
   if (tid < O::SIZE) s1[tid] = o1;
   // the FP64 base of the final stages is absolute; FP32 stage states hold the
   // energy less Phys::eOff
-  const bool base64 = FIN || (VIS && a.mode >= 2);
+  constexpr bool base64 = FIN;
   if (hasS) {
     // Us = base - rkPrev * rprev * dt / detJ: the previous stage's update
     // (the expression of step (4)), evaluated here instead of stored
@@ -1064,17 +947,7 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
     // Final update (mode 2): the earlier stages' terms are subtracted from
     // the base now (after the stage state above used it), in stage order as
     // at the update
-    if (a.mode == 2) {
-      const double dtJ = pdt / pdet;
-#pragma unroll
-      for (int k = 0; k < NF; k++) {
-        double u = pb[k];
-        if (a.nprev > 0) u -= a.c0 * (double)pd[0][k] * dtJ;
-        if (a.nprev > 1) u -= a.c1 * (double)pd[1][k] * dtJ;
-        if (a.nprev > 2) u -= a.c2 * (double)pd[2][k] * dtJ;
-        pb[k] = u;
-      }
-    }
+    if (a.mode == 2) subtractEarlier<NF, T>(a, pd, pdt / pdet, pb);
   }
   __syncthreads();
 
@@ -1084,18 +957,29 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
 #pragma unroll
     for (int r = 0; r < NQ; r++) {
       const int q = fq(r);
+      T uo[NF];
+      if constexpr (MFF) {
+        if (act) {
+          T own[NF];
+#pragma unroll
+          for (int k = 0; k < NF; k++) own[k] = r == 0 ? sU[slot][k][tP] : (T)0;
+          mfmaFaceRound<NF, G::NSP, T>(s1, &sU[slot][0][0], t, own, r, uo);
+        }
+      }
       if (act && q < NFP) {
-        int base, stride, side, dn;
-        fptLine<D, P>(q, base, stride, side, dn);
-        const int lb = padIdx<P>(base), ls = padStride<P>(stride);
-        const T *l1 = s1 + (side ? O::LR : O::LL);
-        T uo[NF], un[NF], dUc[NF];
+        T un[NF], dUc[NF];
+        if constexpr (!MFF) {
+          int base, stride, side, dn;
+          fptLine<D, P>(q, base, stride, side, dn);
+          const int lb = padIdx<P>(base), ls = padStride<P>(stride);
+          const T *l1 = s1 + (side ? O::LR : O::LL);
 #pragma unroll
-        for (int k = 0; k < NF; k++) {
-          T acc = (T)0;
+          for (int k = 0; k < NF; k++) {
+            T acc = (T)0;
 #pragma unroll
-          for (int m = 0; m < P1; m++) acc += l1[m] * sU[slot][k][lb + m * ls];
-          uo[k] = acc;
+            for (int m = 0; m < P1; m++) acc += l1[m] * sU[slot][k][lb + m * ls];
+            uo[k] = acc;
+          }
         }
         const int fi = pfi[r];
         const bool bnd = BND && fi >= FINFO_BOUNDARY;
@@ -1137,7 +1021,12 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
   // along d (calcDivF_spts) and its extrapolation to the two faces normal to d
   // (extrapolateNormalFlux), stored negated as the start of the jump
   if constexpr (MF) {
-    if (act) mfmaAxes<NF, T, FOLD>(sm, slot, t, pJ, F, div, DBG ? a.dbgF + (size_t)e * D * NF * NS : nullptr);
+    if constexpr (FOLD) {
+      if (act) mfmaDivergence<NF, T>(s1, t, pJ, F, div);
+      elementSync<TPE>();
+    } else {
+      if (act) mfmaAxes<NF, T>(sm, slot, t, pJ, F, div, a.dbgF + (size_t)e * D * NF * NS);
+    }
   } else {
 #pragma unroll
     for (int d = 0; d < D; d++) {
@@ -1287,9 +1176,10 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
       // the right element's points keep theirs (face.cpp:74-80)
       if (a.waveSp && hasWs && !right) a.waveSp[(size_t)e * NFP + q] = (double)ws;
       if constexpr (VIS) {
-        // the viscous common flux of this point (k_vflux, before this launch)
+        // the common flux of this point, inviscid and viscous: both sides' shares
+        const T *Gn = a.Gv + (bnd ? 0 : (size_t)pnb[r] * NF * NFP + neighbourFpt<D, P>(q, fi));
 #pragma unroll
-        for (int k = 0; k < NF; k++) Fn[k] += a.Fv[((size_t)e * NF + k) * NFP + q];
+        for (int k = 0; k < NF; k++) Fn[k] = a.Gv[((size_t)e * NF + k) * NFP + q] + (bnd ? (T)0 : Gn[k * NFP]);
       }
       const T scale = right ? -dA : dA;
 #pragma unroll
@@ -1304,109 +1194,23 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
   }
   elementSync<TPE>();
 
-  // (4) correction of the jump (correctDivFlux, solver.cpp:789-806) and the
-  // stage update; the updated state goes to sFd (free after (2)) for its
-  // traces, so that sU keeps the stage state other elements of the block read
-  T utv[NF];  // the updated state at this thread's point, for the traces of (5)
-  if (hasS) {
-    int cq[NFACE], cside[NFACE], cax[NFACE];
-    corrEntries<D, P>(t, cq, cside, cax);
-    T cw[NFACE];  // correction weights, read once for all fields
-#pragma unroll
-    for (int f = 0; f < NFACE; f++) cw[f] = s1[(cside[f] ? O::GR : O::GL) + cax[f]];
-    const size_t eo = (size_t)e * NF * NS;
-#pragma unroll
-    for (int k = 0; k < NF; k++) {
-      T corr = (T)0;
-#pragma unroll
-      for (int f = 0; f < NFACE; f++) corr += cw[f] * sJ[slot][k][cq[f]];
-      const T dv = corr + div[k];
-      const size_t gi = eo + (size_t)k * NS + t;
-      if (a.divF) __builtin_nontemporal_store(dv, a.divF + gi);
-      if (M01 && a.mode == 0) continue;
-      // stage terms RK * divF / detJ * dt, with dt / detJ formed once per point
-      const double dtJ = pdt / pdet;
-      double u = pb[k];
-      // DEF: the base state read again here instead of kept in registers
-      if constexpr (DEF) u = (double)a.UbaseT[gi];
-      if (M23 && a.mode == 2) {
-        // earlier residuals: already subtracted from pb (FIN, before the barrier) or
-        // read here (viscous variant)
-        if constexpr (!FIN) {
-          const T r0 = (a.nprev > 0) ? a.dprev0[gi] : (T)0;
-          const T r1 = (a.nprev > 1) ? a.dprev1[gi] : (T)0;
-          const T r2 = (a.nprev > 2) ? a.dprev2[gi] : (T)0;
-          if (a.nprev > 0) u -= a.c0 * (double)r0 * dtJ;
-          if (a.nprev > 1) u -= a.c1 * (double)r1 * dtJ;
-          if (a.nprev > 2) u -= a.c2 * (double)r2 * dtJ;
-        }
-        const double cl = (a.nprev == 0) ? a.c0 : (a.nprev == 1) ? a.c1 : (a.nprev == 2) ? a.c2 : a.c3;
-        u -= cl * (double)dv * dtJ;
-      } else {
-        u = u - a.rk * (double)dv * dtJ;
-      }
-      // the updated state in the residual precision, for the traces: FP32
-      // states hold the energy less Phys::eOff, and the final stages' FP64
-      // base (hence u) is absolute
-      double ut = u;
-      if constexpr (hasEnergyOffset<T>())
-        if (k == NF - 1 && base64) ut = u - a.ph.eOff;
-      if (!M23 || (M01 && a.mode == 1)) {
-        if (a.Unext) __builtin_nontemporal_store((T)u, a.Unext + gi);
-      } else {
-        __builtin_nontemporal_store(u, a.Uout + gi);
-        if (a.Uout32) __builtin_nontemporal_store((float)ut, a.Uout32 + gi);
-      }
-      sFd[slot][k][tP] = (T)ut;
-      utv[k] = (T)ut;
-    }
-  }
-  if (M01 && a.mode == 0) return;
-  elementSync<TPE>();
-
-  // (5) face traces of the updated state for the next stage, for the faces
-  // whose neighbour is in another block
-  if (act) {
-    T *Fe = a.UfOut + (size_t)e * NF * NFP;
-#pragma unroll
-    for (int r = 0; r < NQ; r++) {
-      const int q = fq(r);
-      T tv[NF];
-      if constexpr (MFF) mfmaFaceRound<NF, G::NSP, T>(s1, &sFd[slot][0][0], t, utv, r, tv);
-      if (q >= NFP) continue;
-      if (!VIS && (pnb[r] < 0 || inBlock(pnb[r]))) continue;
-      if constexpr (MFF) {
-#pragma unroll
-        for (int k = 0; k < NF; k++) __builtin_nontemporal_store(tv[k], Fe + k * NFP + q);
-        continue;
-      }
-      int base, stride, side, dn;
-      fptLine<D, P>(q, base, stride, side, dn);
-      const int lb = padIdx<P>(base), ls = padStride<P>(stride);
-      const T *l1 = s1 + (side ? O::LR : O::LL);
-#pragma unroll
-      for (int k = 0; k < NF; k++) {
-        T acc = (T)0;
-#pragma unroll
-        for (int m = 0; m < P1; m++) acc += l1[m] * sFd[slot][k][lb + m * ls];
-        __builtin_nontemporal_store(acc, Fe + k * NFP + q);
-      }
-    }
-  }
+  // (4) correction of the jump and the stage update, (5) the traces of the
+  // updated state for the faces whose neighbour is in another block; the
+  // updated state goes to sFd (free after (2)), so that sU keeps the stage
+  // state other elements of the block read
+  stageUpdate<D, P, NF, T, FIN, DEF, L>(a, s1, &sJ[slot][0][0], &sFd[slot][0][0], e, t, act, div, pb, pdet, pdt,
+                                        [&](int r) { return VIS || !(pnb[r] < 0 || inBlock(pnb[r])); });
 }
 
 // The inviscid final-stage variant asks for 3 waves per SIMD (at most 168
 // VGPRs): it holds the most prefetched data, and at 2 waves per SIMD the
 // final stage ran 12 % longer.  So do the hex P3 variants with the MFMA
 // contractions, whose accumulators would otherwise take them to 2 waves.
-// The viscous variant runs one wave per SIMD, except the FP64 hex P3 one,
-// whose matrix-core gradient and line operators fit two without spilling.
-template <int D, int P, int NF, typename T, bool BND, bool VIS, bool FIN, int GM = 0>
+template <int D, int P, int NF, typename T, bool BND, bool FIN, int GM = 0>
 __global__ __launch_bounds__((ElemGeo<D, P>::NTH),
-                             (VIS ? ((FR_MFMA && D == 3 && P == 3 && sizeof(T) == 8) ? 2 : 1)
-                              : (FR_MFMA && D == 3 && P == 3) ? (FIN ? FR_MF_FIN_WAVES : FR_MF_WAVES)
-                              : FIN                           ? 3
-                                                              : FR_STAGE_MINW)) void k_stage(StageArgs<T> a) {
+                             ((FR_MFMA && D == 3 && P == 3) ? (FIN ? FR_MF_FIN_WAVES : FR_MF_WAVES)
+                              : FIN                          ? 3
+                                                             : FR_STAGE_MINW)) void k_stage(StageArgs<T> a) {
   __shared__ StageSmem<D, P, NF, T> sm;
   // Workgroups are dealt to the 8 XCDs in turn; remap so that each XCD walks a
   // contiguous range of elements and face neighbours share its L2.  The host
@@ -1415,7 +1219,7 @@ __global__ __launch_bounds__((ElemGeo<D, P>::NTH),
   // in the memory-side cache).
   const int R = gridDim.x >> 3, j = blockIdx.x >> 3;
   const int b = (blockIdx.x & 7) * R + (a.rev ? R - 1 - j : j);
-  stageBody<D, P, NF, T, BND, VIS, FIN, GM>(a, b, sm, (int)threadIdx.x);
+  stageBody<D, P, NF, T, BND, false, FIN, GM>(a, b, sm, (int)threadIdx.x);
 }
 
 // The residual evaluation (mode 0) with the debug outputs of StageArgs

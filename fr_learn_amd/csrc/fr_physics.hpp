@@ -405,94 +405,61 @@ __device__ __forceinline__ void viscousFlux(const Phys &ph, const T *U, const TG
 #pragma unroll
     for (int d = 0; d < D; d++) Fv[d][0] = -(T)ph.diffD * g[d][0];
   } else {
-    // FP64: one reciprocal of rho (recip) for the reference's divisions by
-    // rho; other types (FP32, the adjoint's dual numbers) divide, which is
-    // cheaper for them
-    const T rho = U[0];
-    const T ri = (sizeof(T) == 8) ? recip(rho) : (T)0;
-    auto over = [&](const T &x) -> T {
-      if constexpr (sizeof(T) == 8) return x * ri;
-      else return x / rho;
-    };
-    const T u = over(U[1]), v = over(U[2]);
-    T e = over(U[D + 1]) - (T)0.5 * (u * u + v * v);
-    T w = (T)0;
-    if constexpr (D == 3) {
-      w = over(U[3]);
-      e -= (T)0.5 * (w * w);
-    }
-    const TG dRho_dx = g[0][0], dRhoU_dx = g[0][1], dRhoV_dx = g[0][2], dE_dx = g[0][D + 1];
-    const TG dRho_dy = g[1][0], dRhoU_dy = g[1][1], dRhoV_dy = g[1][2], dE_dy = g[1][D + 1];
-    TG dRho_dz = 0, dRhoU_dz = 0, dRhoV_dz = 0, dRhoW_dx = 0, dRhoW_dy = 0, dRhoW_dz = 0, dE_dz = 0;
-    if constexpr (D == 3) {
-      dRho_dz = g[2][0];
-      dRhoU_dz = g[2][1];
-      dRhoV_dz = g[2][2];
-      dRhoW_dx = g[0][3];
-      dRhoW_dy = g[1][3];
-      dRhoW_dz = g[2][3];
-      dE_dz = g[2][4];
-    }
+    // Written for few operations: one reciprocal of rho for the reference's
+    // divisions, the velocity gradients (grad m - v grad rho) / rho, and the
+    // energy gradient from that of the total energy,
+    //   grad e = (grad E - (E / rho) grad rho) / rho - sum_c v_c grad v_c,
+    // which is the reference's grad E - grad(rho |v|^2 / 2) - e grad rho
+    // regrouped; the ratio gamma / Pr and the third of the divergence are
+    // constants.  Ulp-level differences.
+    const T ri = recip(U[0]);
+    T v[D];
+#pragma unroll
+    for (int c = 0; c < D; c++) v[c] = U[c + 1] * ri;
+    const T H = U[D + 1] * ri;
     T mu = (T)ph.mu_inf;
     if (!ph.fixVis) {  // Sutherland's law
-      const T rt = ((T)ph.gamma - (T)1.0) * e / (T)ph.rt_inf;
+      T q = v[0] * v[0];
+#pragma unroll
+      for (int c = 1; c < D; c++) q += v[c] * v[c];
+      const T rt = ((T)ph.gamma - (T)1.0) * (H - (T)0.5 * q) / (T)ph.rt_inf;
       mu *= pow(rt, (T)1.5) * ((T)1. + (T)ph.c_sth) / (rt + (T)ph.c_sth);
     }
-    const T du_dx = over(dRhoU_dx - dRho_dx * u), du_dy = over(dRhoU_dy - dRho_dy * u);
-    const T dv_dx = over(dRhoV_dx - dRho_dx * v), dv_dy = over(dRhoV_dy - dRho_dy * v);
-    T du_dz = 0, dv_dz = 0, dw_dx = 0, dw_dy = 0, dw_dz = 0;
+    const T mr = mu * ri;  // mu / rho: the stresses need mu grad v
+    // G[d][c] = mu dv_c/dx_d and h[d] = mu de/dx_d
+    T G[D][D], h[D];
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+#pragma unroll
+      for (int c = 0; c < D; c++) G[d][c] = mr * (g[d][c + 1] - v[c] * g[d][0]);
+      h[d] = mr * (g[d][D + 1] - H * g[d][0]);
+#pragma unroll
+      for (int c = 0; c < D; c++) h[d] -= v[c] * G[d][c];
+    }
+    T diag = G[0][0] + G[1][1];
+    if constexpr (D == 3) diag += G[2][2];
+    diag = diag * (T)(1.0 / 3.0);
+    const T kq = (T)(ph.gamma / ph.prandtl);
+    T tau[D][D];  // tau[d][c], symmetric
+#pragma unroll
+    for (int d = 0; d < D; d++) tau[d][d] = (T)2.0 * (G[d][d] - diag);
+    tau[0][1] = tau[1][0] = G[1][0] + G[0][1];
     if constexpr (D == 3) {
-      du_dz = over(dRhoU_dz - dRho_dz * u);
-      dv_dz = over(dRhoV_dz - dRho_dz * v);
-      dw_dx = over(dRhoW_dx - dRho_dx * w);
-      dw_dy = over(dRhoW_dy - dRho_dy * w);
-      dw_dz = over(dRhoW_dz - dRho_dz * w);
+      tau[0][2] = tau[2][0] = ph.viscFix ? G[2][0] + G[0][2] : G[2][0] + G[0][1];
+      tau[1][2] = tau[2][1] = ph.viscFix ? G[2][1] + G[1][2] : G[2][0] + G[1][1];
     }
-    T dK_dx, dK_dy, dK_dz = 0;
-    if constexpr (D == 2) {
-      dK_dx = (T)0.5 * (u * u + v * v) * dRho_dx + rho * (u * du_dx + v * dv_dx);
-      dK_dy = (T)0.5 * (u * u + v * v) * dRho_dy + rho * (u * du_dy + v * dv_dy);
-    } else {
-      dK_dx = (T)0.5 * (u * u + v * v + w * w) * dRho_dx + rho * (u * du_dx + v * dv_dx + w * dw_dx);
-      dK_dy = (T)0.5 * (u * u + v * v + w * w) * dRho_dy + rho * (u * du_dy + v * dv_dy + w * dw_dy);
-      dK_dz = (T)0.5 * (u * u + v * v + w * w) * dRho_dz + rho * (u * du_dz + v * dv_dz + w * dw_dz);
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      T q = kq * h[d];
+#pragma unroll
+      for (int c = 0; c < D; c++) q += v[c] * tau[d][c];
+      Fv[d][0] = (T)0.0;
+#pragma unroll
+      for (int c = 0; c < D; c++) Fv[d][c + 1] = -tau[d][c];
+      Fv[d][D + 1] = -q;
     }
-    const T de_dx = over(dE_dx - dK_dx - dRho_dx * e);
-    const T de_dy = over(dE_dy - dK_dy - dRho_dy * e);
-    T de_dz = 0;
-    if constexpr (D == 3) de_dz = over(dE_dz - dK_dz - dRho_dz * e);
-    const T diag = (du_dx + dv_dy + dw_dz) / (T)3.0;
-    const T tauxx = (T)2.0 * mu * (du_dx - diag), tauyy = (T)2.0 * mu * (dv_dy - diag);
-    const T tauxy = mu * (du_dy + dv_dx);
-    T tauxz = 0, tauyz = 0, tauzz = 0;
-    if constexpr (D == 3) {
-      if (ph.viscFix) {
-        tauxz = mu * (du_dz + dw_dx);
-        tauyz = mu * (dv_dz + dw_dy);
-      } else {
-        tauxz = mu * (du_dz + dv_dx);
-        tauyz = mu * (du_dz + dv_dy);
-      }
-      tauzz = (T)2.0 * mu * (dw_dz - diag);
-    }
-    const T kq = (mu / (T)ph.prandtl) * (T)ph.gamma;
-    Fv[0][0] = (T)0.0;
-    Fv[0][1] = -tauxx;
-    Fv[0][2] = -tauxy;
-    Fv[0][D + 1] = -(u * tauxx + v * tauxy + w * tauxz + kq * de_dx);
-    Fv[1][0] = (T)0.0;
-    Fv[1][1] = -tauxy;
-    Fv[1][2] = -tauyy;
-    Fv[1][D + 1] = -(u * tauxy + v * tauyy + w * tauyz + kq * de_dy);
-    if constexpr (D == 3) {
-      Fv[0][3] = ph.viscFix ? -tauxz : -tauzz;
-      Fv[1][3] = -tauyz;
-      Fv[2][0] = (T)0.0;
-      Fv[2][1] = -tauxz;
-      Fv[2][2] = -tauyz;
-      Fv[2][3] = -tauzz;
-      Fv[2][4] = -(u * tauxz + v * tauyz + w * tauzz + kq * de_dz);
-    }
+    if constexpr (D == 3)
+      if (!ph.viscFix) Fv[0][3] = -tau[2][2];
   }
 }
 
@@ -535,6 +502,59 @@ __device__ __forceinline__ T ldgPenalty(const Phys &ph, const T *n) {
     pen = -(T)ph.penFact;
   }
   return pen;
+}
+
+// Fields with a viscous flux: all but the mass of Navier-Stokes (fields
+// NF - viscFields .. NF - 1).
+template <int NF>
+constexpr int viscFields() {
+  return NF == 1 ? 1 : NF - 1;
+}
+
+// The weights w of one side's viscous flux F in the LDG common normal flux
+// sum_d Fc[d] n[d] (face::calcViscousFlux, face.cpp:177-287), the same for
+// every field: with Fc[d] = (FL + FR)[d] / 2 + pen n[d] n.(FL - FR), the left
+// side enters with w = n / 2 + pen |n|^2 n and the right one with
+// n / 2 - pen |n|^2 n; face.cpp:245 takes F_L,y for F_L,z in n.(FL - FR)
+// (viscFix = 0).  Boundaries take one side's flux alone (w = n), and
+// advection-diffusion the central flux of -diffD grad u (face.cpp:270-279;
+// its boundaries a zero outside gradient).  n is the left element's normal.
+template <int D, int NF, typename T>
+__device__ __forceinline__ void ldgWeights(const Phys &ph, bool bnd, bool right, const T *n, T *w) {
+  if constexpr (NF == 1) {
+#pragma unroll
+    for (int d = 0; d < D; d++) w[d] = (T)0.5 * n[d];
+  } else {
+    T nn = n[0] * n[0];
+#pragma unroll
+    for (int d = 1; d < D; d++) nn += n[d] * n[d];
+    const T pn = ldgPenalty<D, T>(ph, n) * nn;
+#pragma unroll
+    for (int d = 0; d < D; d++) w[d] = bnd ? n[d] : (T)0.5 * n[d] + (right ? -pn * n[d] : pn * n[d]);
+    if constexpr (D == 3)
+      if (!bnd && !right && !ph.viscFix) {
+        w[1] += pn * n[2];
+        w[2] -= pn * n[2];
+      }
+  }
+}
+
+// One side's share of the viscous common normal flux, w . F_v(U, g), for the
+// fields that have one (viscFields).
+template <int D, int NF, typename T>
+__device__ __forceinline__ void viscousShare(const Phys &ph, bool bnd, bool right, const T *U, const T g[D][NF],
+                                             const T *n, T *C) {
+  constexpr int NV = viscFields<NF>();
+  T F[D][NF], w[D];
+  viscousFlux<D, NF, T>(ph, U, g, F);
+  ldgWeights<D, NF, T>(ph, bnd, right, n, w);
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+    T acc = w[0] * F[0][NF - NV + k];
+#pragma unroll
+    for (int d = 1; d < D; d++) acc += w[d] * F[d][NF - NV + k];
+    C[k] = acc;
+  }
 }
 
 // Adds the common LDG viscous normal flux sum_d Fc[d] n[d] to the inviscid

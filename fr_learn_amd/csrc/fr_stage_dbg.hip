@@ -1,13 +1,13 @@
 // fr_stage_dbg.hip -- the debug residual evaluation behind fr_get_array: the
-// stage kernel with its debug outputs (k_stage_dbg), after the gradient and
-// viscous-flux kernels on the viscous path, FP64 quads and hexes.  Its own
+// stage kernel with its debug outputs (k_stage_dbg), after k_visc_flux on the
+// viscous path, FP64 quads and hexes.  Its own
 // translation unit, so that these instances compile beside the production
 // ones.
 #include "fr_stage_impl.hpp"
 
 namespace frimpl {
 
-int launchStageDbg(fr_ctx *c, const frdev::StageArgs<double> &a, double *dUs) {
+int launchStageDbg(fr_ctx *c, const frdev::StageArgs<double> &a, double *dUf, double *dUs) {
   if (c->tri || c->prec != FR_PREC_FP64) return fail(FR_EINVAL, "debug residual: FP64 quads and hexes only");
   const bool bnd = c->conn.nIntFaces < (int)c->conn.faces.size();
   const bool vis = c->cfg.viscous != 0;
@@ -17,19 +17,11 @@ int launchStageDbg(fr_ctx *c, const frdev::StageArgs<double> &a, double *dUs) {
     using G = frdev::ElemGeo<D, P>;
     const unsigned nb = (unsigned)(((c->nE + G::EPB - 1) / G::EPB + 7) / 8 * 8);
     if (vis) {
-      frdev::GradArgs<double> g{a.Uin,  a.UfIn,  a.JG,   a.detJ,  a.fgeo, a.fnbr,
-                                a.finfo, a.oned, (double *)c->dUf, a.nEles, a.ph, a.affine, dUs};
-      if (bnd) hipLaunchKernelGGL((frdev::k_grad<D, P, NF, double, true>), dim3(nb), dim3(G::NTH), 0, c->stream, g);
-      else hipLaunchKernelGGL((frdev::k_grad<D, P, NF, double, false>), dim3(nb), dim3(G::NTH), 0, c->stream, g);
-      const unsigned nq = (unsigned)(((long)c->nE * G::NFP + 255) / 256);
-      if (bnd)
-        hipLaunchKernelGGL((frdev::k_vflux<D, P, NF, double, true>), dim3(nq), dim3(256), 0, c->stream, a.UfIn,
-                           (const double *)c->dUf, a.fgeo, a.fnbr, a.finfo, a.affine, a.ph, a.nEles,
-                           (double *)a.Fv);
-      else
-        hipLaunchKernelGGL((frdev::k_vflux<D, P, NF, double, false>), dim3(nq), dim3(256), 0, c->stream, a.UfIn,
-                           (const double *)c->dUf, a.fgeo, a.fnbr, a.finfo, a.affine, a.ph, a.nEles,
-                           (double *)a.Fv);
+      constexpr int OUT = frdev::VISC_SHARES | frdev::VISC_GRADIENT;
+      if (bnd) hipLaunchKernelGGL((frdev::k_visc_flux<D, P, NF, double, true, OUT>), dim3(nb), dim3(G::NTH), 0,
+                                  c->stream, a, dUf, dUs);
+      else hipLaunchKernelGGL((frdev::k_visc_flux<D, P, NF, double, false, OUT>), dim3(nb), dim3(G::NTH), 0,
+                              c->stream, a, dUf, dUs);
       if ((err = hipGetLastError()) != hipSuccess) return;
       if (bnd) hipLaunchKernelGGL((frdev::k_stage_dbg<D, P, NF, true, true>), dim3(nb), dim3(G::NTH), 0, c->stream, a);
       else hipLaunchKernelGGL((frdev::k_stage_dbg<D, P, NF, false, true>), dim3(nb), dim3(G::NTH), 0, c->stream, a);

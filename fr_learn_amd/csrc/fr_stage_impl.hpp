@@ -1,14 +1,14 @@
-// fr_stage_impl.hpp -- launches of the stage kernel (and, on the viscous path,
-// the gradient kernel before it); instantiated per precision in
+// fr_stage_impl.hpp -- launches of the stage kernel (on the viscous path, of its
+// two kernels); instantiated per precision in
 // fr_stage64.hip and fr_stage32.hip so that the two compile in parallel.
 #pragma once
 
 #include "fr_ctx.hpp"
+#include "fr_viscous.hpp"
 
 namespace frimpl {
 
-// Launch of the stage kernel variant for `mode` with arguments `a` (and the
-// gradient kernel before it on the viscous path), quads (DD = 2) or hexes
+// Launch of the stage kernel variant for `mode` with arguments `a`, quads (DD = 2) or hexes
 // (DD = 3); the four (precision, DD) instances compile in their own
 // translation units (fr_stage{64,32}_{2,3}d.hip).
 template <typename T, int DD>
@@ -26,32 +26,29 @@ int launchStageArgsD(fr_ctx *c, const frdev::StageArgs<T> &a, int mode) {
     // grid padded to a multiple of the 8 XCDs (the kernels remap block ids)
     const unsigned nb = (unsigned)(((c->nE + G::EPB - 1) / G::EPB + 7) / 8 * 8);
     if (vis) {
-      frdev::GradArgs<T> g{a.Uin,  a.UfIn,  a.JG,   a.detJ,  a.fgeo, a.fnbr,
-                            a.finfo, a.oned, (T *)c->dUf, a.nEles, a.ph, a.affine, nullptr};
       {
         TimeScope ts(c, 3);
-        if (bnd) hipLaunchKernelGGL((frdev::k_grad<D, P, NF, T, true>), dim3(nb), dim3(G::NTH), 0, c->stream, g);
-        else hipLaunchKernelGGL((frdev::k_grad<D, P, NF, T, false>), dim3(nb), dim3(G::NTH), 0, c->stream, g);
-        const unsigned nq = (unsigned)(((long)c->nE * G::NFP + 255) / 256);
-        if (bnd)
-          hipLaunchKernelGGL((frdev::k_vflux<D, P, NF, T, true>), dim3(nq), dim3(256), 0, c->stream, a.UfIn,
-                             (const T *)c->dUf, a.fgeo, a.fnbr, a.finfo, a.affine, a.ph, a.nEles, (T *)a.Fv);
-        else
-          hipLaunchKernelGGL((frdev::k_vflux<D, P, NF, T, false>), dim3(nq), dim3(256), 0, c->stream, a.UfIn,
-                             (const T *)c->dUf, a.fgeo, a.fnbr, a.finfo, a.affine, a.ph, a.nEles, (T *)a.Fv);
+        if (bnd) hipLaunchKernelGGL((frdev::k_visc_flux<D, P, NF, T, true>), dim3(nb), dim3(G::NTH), 0, c->stream, a,
+                                    (T *)nullptr, (T *)nullptr);
+        else hipLaunchKernelGGL((frdev::k_visc_flux<D, P, NF, T, false>), dim3(nb), dim3(G::NTH), 0, c->stream, a,
+                                (T *)nullptr, (T *)nullptr);
       }
       if ((err = hipGetLastError()) != hipSuccess) return;
       TimeScope ts(c, 0);
-      if (bnd) hipLaunchKernelGGL((frdev::k_stage<D, P, NF, T, true, true, false>), dim3(nb), dim3(G::NTH), 0,
-                                  c->stream, a);
-      else hipLaunchKernelGGL((frdev::k_stage<D, P, NF, T, false, true, false>), dim3(nb), dim3(G::NTH), 0,
-                              c->stream, a);
+      auto launch = [&](auto Bc, auto Fc) {
+        hipLaunchKernelGGL((frdev::k_visc_update<D, P, NF, T, decltype(Bc)::value, decltype(Fc)::value>), dim3(nb),
+                           dim3(G::NTH), 0, c->stream, a);
+      };
+      if (bnd && mode >= 2) launch(std::true_type{}, std::true_type{});
+      else if (bnd) launch(std::true_type{}, std::false_type{});
+      else if (mode >= 2) launch(std::false_type{}, std::true_type{});
+      else launch(std::false_type{}, std::false_type{});
     } else {
       TimeScope ts(c, 0);
       // the inviscid variants: boundary faces or not, final stage or not,
       // geometry from the stored arrays or from the nodal map (GM)
       auto launch = [&](auto Bc, auto Fc, auto Gc) {
-        hipLaunchKernelGGL((frdev::k_stage<D, P, NF, T, decltype(Bc)::value, false, decltype(Fc)::value,
+        hipLaunchKernelGGL((frdev::k_stage<D, P, NF, T, decltype(Bc)::value, decltype(Fc)::value,
                                            decltype(Gc)::value>),
                            dim3(nb), dim3(G::NTH), 0, c->stream, a);
       };

@@ -56,14 +56,6 @@ struct TriSmem {
   T sN[G::EPB][NF][G::NS];     // updated state
 };
 
-// Reference unit normal of the edge of flux point q (edges v0v1, v1v2, v2v0).
-template <typename T>
-__device__ __forceinline__ void triNormal(int f, T &nx, T &ny) {
-  const T h = (T)0.70710678118654752440;
-  nx = (f == 0) ? (T)0 : (f == 1) ? h : (T)-1;
-  ny = (f == 0) ? (T)-1 : (f == 1) ? h : (T)0;
-}
-
 // The loads of one thread of a triangle's stage (element ec): at its
 // solution point tc the metrics, detJ and base state, the element's time
 // step; at its flux point qc the face record, normal, dA and the neighbour's
@@ -178,7 +170,7 @@ struct TriPoint {
 };
 
 // One RK stage of element block b (EPB elements) with the arguments a, the
-// operator products as each thread's line sums (FP32).  With FR_FOLD the
+// operator products as each thread's line sums (FP32).  The
 // divergence operators are the folded ones (TriGeo::DRF, DSF, copied into the
 // table's Dr and Ds places) and the jump is the common flux alone.
 template <int P, int NF, typename T, bool BND, bool FIN, int LAY = 0>
@@ -193,7 +185,7 @@ __device__ __forceinline__ void triStageBody(const StageArgs<T> &a, const int b,
   const size_t ec = (size_t)(act ? e : a.nEles - 1);
   const int tc = t < NS ? t : NS - 1, qc = t < NFP ? t : NFP - 1;
 
-  for (int i = tid; i < G::TAB; i += 256) sm.tab[i] = a.oned[(FR_FOLD && i < 2 * NS * NS) ? G::DRF + i : i];
+  for (int i = tid; i < G::TAB; i += 256) sm.tab[i] = a.oned[(i < 2 * NS * NS) ? G::DRF + i : i];
   if (act)
     for (int i = t; i < NF * NS; i += TPE) (&sm.sU[slot][0][0])[i] = a.Uin[ec * NF * NS + i];
   const TriPoint<P, NF, T, BND, FIN> pt(a, ec, tc, qc);
@@ -226,28 +218,10 @@ __device__ __forceinline__ void triStageBody(const StageArgs<T> &a, const int b,
     pt.normalFlux(a.ph, uo, Fn);
   }
   elementSync<TPE>();
-  // (2) jump at the flux point: Fn dA - (E F~) . tNorm, or Fn dA alone with
-  // the folded divergence operators
-  if (FR_FOLD && hasQ) {
+  // (2) jump at the flux point: Fn dA alone, with the folded operators
+  if (hasQ) {
 #pragma unroll
     for (int k = 0; k < NF; k++) sm.sJ[slot][k][t] = Fn[k];
-  } else if (hasQ) {
-    T tx, ty;
-    triNormal<T>(t / NFPF, tx, ty);
-    T fr[NF], fs[NF];
-#pragma unroll
-    for (int k = 0; k < NF; k++) fr[k] = fs[k] = (T)0;
-#pragma unroll 3
-    for (int s = 0; s < NS; s++) {
-      const T w = Em[t * NS + s];
-#pragma unroll
-      for (int k = 0; k < NF; k++) {
-        fr[k] += w * sm.sF[slot][0][k][s];
-        fs[k] += w * sm.sF[slot][1][k][s];
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < NF; k++) sm.sJ[slot][k][t] = Fn[k] - (tx * fr[k] + ty * fs[k]);
   }
   elementSync<TPE>();
   // (3) divergence + correction, stage update (as k_stage phase 4)
