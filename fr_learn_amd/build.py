@@ -19,7 +19,7 @@ SOURCES = ["fr_stage64_3d.hip", "fr_stage32_3d.hip", "fr_stage_dbg.hip", "fr_adj
            "fr_batch.hip", "fr_adjoint_v3ad.hip", "fr_api.hip", "fr_host.cpp", "fr_output.cpp", "fr_tri_ops.cpp",
            "fr_tri.hip", "fr_error.hip"]
 HEADERS = ["fr_ctx.hpp", "fr_host.hpp", "fr_kernels.hpp", "fr_layout.hpp", "fr_physics.hpp", "fr_adjoint.hpp",
-           "fr_adjoint_vis.hpp", "fr_dual.hpp", "fr_batch.hpp", "fr_stage_impl.hpp", "fr_tri.hpp", "fr_viscous.hpp"]
+           "fr_adjoint_vis.hpp", "fr_dual.hpp", "fr_batch.hpp", "fr_stage_impl.hpp", "fr_tri.hpp", "fr_viscous.hpp", "fr_reverse.hpp"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

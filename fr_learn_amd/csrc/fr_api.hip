@@ -28,10 +28,11 @@ void freeAll(fr_ctx *c) {
   void *bufs[] = {c->U,       c->U0,      c->detJ,    c->JG64,    c->fgeo64, c->ownN,  c->wts,
                   c->oned64,  c->part,    c->U32,     c->JG32,    c->fgeo32, c->oned32, c->Us,
                   c->Uf[0],   c->Uf[1],   c->divF[0], c->divF[1], c->divF[2], c->divF[3], c->fnbr,
-                  c->finfo,   c->Gv,      c->dtG,     c->dtE,     c->adjA,   c->adjTr, c->adjTr2,
-                  c->adjLam,  c->adjOut,  c->adjNu,   c->adjW[0], c->adjW[1], c->adjS[0], c->adjS[1],
-                  c->adjS[2], c->adjS[3], c->adjQf,   c->adjB,    c->JGc64,  c->detJc, c->fgeoc64,
-                  c->JGc32,   c->fgeoc32, c->adjUo,   c->adjQo,   c->adjCj,   c->waveSp,
+                  c->finfo,   c->Gv,      c->dtG,     c->dtE,     c->adjA[0], c->adjA[1],
+                  c->adjTr[0], c->adjTr[1], c->adjTr[2], c->adjTr[3],
+                  c->adjLam,  c->adjOut,  c->adjNu,   c->adjW,    c->adjS[0], c->adjS[1],
+                  c->adjS[2], c->adjS[3], c->adjB,    c->JGc64,  c->detJc, c->fgeoc64,
+                  c->JGc32,   c->fgeoc32, c->waveSp,
                   c->dtNum,   c->wsurf,   c->dtPart,  c->geoN64,  c->geoN32,  c->errTab, c->Xd};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
@@ -406,45 +407,57 @@ int adjCheck(fr_ctx *c) {
   if (c->tri) return fail(FR_EINVAL, "the adjoint is not available for triangles");
   const size_t nSt = c->nState(), nTr = (size_t)c->nE * c->NF * c->NFP;
   int rc;
-  if (!c->adjA) {
-    if ((rc = dmalloc(&c->adjA, nTr)) || (rc = dmalloc(&c->adjTr, nTr)) || (rc = dmalloc(&c->adjTr2, nTr)) ||
-        (rc = dmalloc(&c->adjLam, nSt)) || (rc = dmalloc(&c->adjOut, nSt)) || (rc = dmalloc(&c->adjNu, nSt)) ||
-        (rc = dmalloc(&c->adjW[0], nSt)) || (rc = dmalloc(&c->adjW[1], nSt)))
+  if (!c->adjB) {
+    if ((!c->adjLam && (rc = dmalloc(&c->adjLam, nSt))) || (!c->adjOut && (rc = dmalloc(&c->adjOut, nSt))) ||
+        (!c->adjNu && (rc = dmalloc(&c->adjNu, nSt))) || (!c->adjW && (rc = dmalloc(&c->adjW, nSt))))
       return rc;
-    for (int s = 1; s < c->nRK; s++)
-      if ((rc = dmalloc(&c->adjS[s], nSt))) return rc;
-    if (c->cfg.viscous && ((rc = dmalloc(&c->adjQf, nTr * c->D)) || (rc = dmalloc(&c->adjB, nTr)) ||
-                           (rc = dmalloc(&c->adjUo, nTr)) || (rc = dmalloc(&c->adjQo, nTr * c->D)) ||
-                           (rc = dmalloc(&c->adjCj, nTr))))
-      return rc;
+    for (int s = 0; s < c->nRK; s++)
+      if ((!c->adjTr[s] && (rc = dmalloc(&c->adjTr[s], nTr))) ||
+          (s > 0 && !c->adjS[s] && (rc = dmalloc(&c->adjS[s], nSt))))
+        return rc;
+    for (int p = 0; p < 2; p++)
+      if (!c->adjA[p] && (rc = dmalloc(&c->adjA[p], nTr))) return rc;
+    // last, so that a context whose allocations failed midway tries again
+    if ((rc = dmalloc(&c->adjB, c->cfg.viscous ? nTr : 1))) return rc;
   }
   return 0;
 }
 
+// The traces of the state Us at every flux point, into tr.
+int fullTraces(fr_ctx *c, const double *Us, double *tr) {
+  dispatch(c->D, c->P, c->NF, [&](auto Dc, auto Pc, auto NFc) {
+    constexpr int D = decltype(Dc)::value, P = decltype(Pc)::value, NF = decltype(NFc)::value;
+    const long nq = (long)c->nE * frdev::ElemGeo<D, P>::NFP;
+    hipLaunchKernelGGL((frdev::k_trace<D, P, NF, double>), dim3(nblk(nq)), dim3(256), 0, c->stream, Us, tr, c->oned64,
+                       c->nE);
+  });
+  HIP_TRY(hipGetLastError());
+  return 0;
+}
+
 // The stage states of one RK step from U (timeStepA, solver.cpp:307-345):
-// S[0] = U, S[s+1] = U - RKa[s+1] R(S[s]) dt / detJ, with the stage kernel.
+// S[0] = U, S[s+1] = U - RKa[s+1] R(S[s]) dt / detJ, with the stage kernel,
+// and their traces in adjTr (each stage launch writes the next state's, all
+// faces of them).
 int stageStates(fr_ctx *c, const double **S) {
   S[0] = c->U;
+  int rc = fullTraces(c, S[0], c->adjTr[0]);
+  if (rc) return rc;
   for (int s = 0; s + 1 < c->nRK; s++) {
-    dispatch(c->D, c->P, c->NF, [&](auto Dc, auto Pc, auto NFc) {
-      constexpr int D = decltype(Dc)::value, P = decltype(Pc)::value, NF = decltype(NFc)::value;
-      const long nq = (long)c->nE * frdev::ElemGeo<D, P>::NFP;
-      hipLaunchKernelGGL((frdev::k_trace<D, P, NF, double>), dim3(nblk(nq)), dim3(256), 0, c->stream, S[s],
-                         c->adjTr, c->oned64, c->nE);
-    });
-    HIP_TRY(hipGetLastError());
     // the update's own arguments, redirected to the adjoint's buffers
     frdev::StageArgs<double> a = makeStageArgs<double>(c, 0, 0, 1, s, c->RKa[s + 1]);
     a.Uin = S[s];
-    a.UfIn = c->adjTr;
-    a.UfOut = c->adjTr2;
+    a.rprev = nullptr;
+    a.UfIn = c->adjTr[s];
+    a.UfOut = c->adjTr[s + 1];
+    a.fullTraces = 1;
     a.divF = nullptr;
     a.divW = c->adjNu;  // written by vjpStepDev after this
     a.Unext = c->adjS[s + 1];
     a.Uout = nullptr;
     a.Uout32 = nullptr;
     a.waveSp = nullptr;  // the recomputation leaves the CFL wave speeds alone
-    int rc = launchStageArgs<double>(c, a, 1);
+    rc = launchStageArgs<double>(c, a, 1);
     if (rc) return rc;
     S[s + 1] = c->adjS[s + 1];
   }
@@ -455,27 +468,48 @@ int stageStates(fr_ctx *c, const double **S) {
 // nu_s = -c_s (dt/detJ) lam1 - RKa[s+1] (dt/detJ) w_{s+1},
 // w_s = (dR/dU at S[s])^T nu_s, lam0 = lam1 + sum_s w_s, where c_s is the
 // weight of R_s in the final update (RKb, or RKa[nRK] on the last stage of
-// the Jameson schemes).
+// the Jameson schemes).  Stage s's last kernel adds w_s to lam0 and forms
+// nu_{s-1} with its face cotangents.
 int vjpStepDev(fr_ctx *c, const double *lam1, double *lam0) {
   const double *S[4];
   int rc = stageStates(c, S);
   if (rc) return rc;
-  const long n = (long)c->nState();
-  HIP_TRY(hipMemcpyAsync(lam0, lam1, n * 8, hipMemcpyDeviceToDevice, c->stream));
-  const double *wNext = nullptr;
+  auto weight = [&](int s) {
+    return (c->cfg.timeType < 5) ? c->RKb[s] : (s == c->nRK - 1 ? c->RKa[c->nRK] : 0.0);
+  };
+  int p = 0;
+  frdev::VjpArgs a = vjpArgs(c, c->U, nullptr, nullptr, nullptr);
+  a.lam1 = lam1;
+  a.lam0 = lam0;
+  a.nuNext = c->adjNu;
+  a.ANext = c->adjA[p];
+  a.alpha = -weight(c->nRK - 1);
+  if ((rc = vjpSeed(c, a))) return rc;
   for (int s = c->nRK - 1; s >= 0; s--) {
-    const double cs = (c->cfg.timeType < 5) ? c->RKb[s] : (s == c->nRK - 1 ? c->RKa[c->nRK] : 0.0);
-    const double an = (s + 1 < c->nRK) ? c->RKa[s + 1] : 0.0;
-    hipLaunchKernelGGL(frdev::k_dtj_combine, dim3(nblk(n)), dim3(256), 0, c->stream, lam1, wNext, c->detJ,
-                       dtSource(c).first, dtSource(c).second, -cs, -an, c->NF, c->NS, n, c->adjNu);
-    HIP_TRY(hipGetLastError());
-    double *w = c->adjW[s & 1];
-    if ((rc = vjpResidualDev(c, S[s], c->adjNu, w))) return rc;
-    hipLaunchKernelGGL(frdev::k_accumulate, dim3(nblk(n)), dim3(256), 0, c->stream, lam0, w, n);
-    HIP_TRY(hipGetLastError());
-    wNext = w;
+    a = vjpArgs(c, S[s], c->adjTr[s], c->adjNu, c->adjA[p]);
+    a.lam1 = lam1;
+    a.lam0 = lam0;
+    if (s > 0) {
+      a.nuNext = c->adjNu;
+      a.ANext = c->adjA[p ^ 1];
+      a.alpha = -weight(s - 1);
+      a.beta = -c->RKa[s];
+    }
+    if ((rc = vjpStage(c, a))) return rc;
+    p ^= 1;
   }
   return 0;
+}
+
+// out = (d divF / dU)^T lam at the state Us (device arrays, device layout)
+int vjpResidualDev(fr_ctx *c, const double *Us, const double *lam, double *out) {
+  int rc = fullTraces(c, Us, c->adjTr[0]);
+  if (rc) return rc;
+  frdev::VjpArgs a = vjpArgs(c, Us, c->adjTr[0], lam, c->adjA[0]);
+  a.ANext = c->adjA[0];
+  if ((rc = vjpSeed(c, a))) return rc;
+  a.out = out;
+  return vjpStage(c, a);
 }
 
 int createImpl(const fr_config *cfg, const fr_mesh *m, int precision, fr_ctx *c) {

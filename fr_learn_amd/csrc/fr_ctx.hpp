@@ -54,6 +54,10 @@ inline unsigned nblk(long n, int b = 256) { return (unsigned)((n + b - 1) / b); 
 
 struct fr_batch;
 
+namespace frdev {
+struct VjpArgs;
+}
+
 struct fr_ctx {
   fr_config cfg{};
   int prec = FR_PREC_FP64;
@@ -107,12 +111,13 @@ struct fr_ctx {
   bool dtFrozen = false;  // the adjoint's replay: dt given, wave speeds untouched
   unsigned gen = 0;       // bumped by every setting the batched launch arguments capture
   std::vector<fr_batch *> batches;  // batches this context is a member of
-  // adjoint work buffers (FP64, allocated on first use)
-  double *adjA = nullptr, *adjTr = nullptr, *adjTr2 = nullptr;  // face cotangents, trace scratch
-  double *adjLam = nullptr, *adjOut = nullptr, *adjNu = nullptr, *adjW[2] = {nullptr, nullptr};
-  double *adjQf = nullptr, *adjB = nullptr;                     // viscous: gradient traces, jump cotangents
-  double *adjUo = nullptr, *adjQo = nullptr, *adjCj = nullptr;  // viscous: face pull-backs, forward jumps
-  double *adjS[4] = {nullptr, nullptr, nullptr, nullptr};       // RK stage states
+  // adjoint work buffers (FP64, allocated on first use): the RK stages' states
+  // and traces, face cotangents (double-buffered from stage to stage), the
+  // step's cotangents, a stage's nu and w, and (viscous) the jumps' cotangents
+  double *adjS[4] = {nullptr, nullptr, nullptr, nullptr};
+  double *adjTr[4] = {nullptr, nullptr, nullptr, nullptr};
+  double *adjA[2] = {nullptr, nullptr};
+  double *adjLam = nullptr, *adjOut = nullptr, *adjNu = nullptr, *adjW = nullptr, *adjB = nullptr;
   int32_t *fnbr = nullptr;
   int8_t *finfo = nullptr;
   size_t partCap = 0;
@@ -226,8 +231,11 @@ int launchStageArgs(fr_ctx *c, const frdev::StageArgs<T> &a, int mode);
 // gradient traces into dUf and the gradient at the spts into dUs),
 // fr_stage_dbg.hip.
 int launchStageDbg(fr_ctx *c, const frdev::StageArgs<double> &a, double *dUf, double *dUs);
-// (d divF / dU)^T lam at the state Us, device arrays (fr_adjoint.hip).
-int vjpResidualDev(fr_ctx *c, const double *Us, const double *lam, double *out);
+// The adjoint of one RK stage and its seed (fr_adjoint.hip): the arguments for
+// the state Us with its traces tr, the cotangent nu and its face cotangents A.
+frdev::VjpArgs vjpArgs(const fr_ctx *c, const double *Us, const double *tr, const double *nu, const double *A);
+int vjpSeed(fr_ctx *c, const frdev::VjpArgs &a);
+int vjpStage(fr_ctx *c, const frdev::VjpArgs &a);
 // triangle kernels (fr_tri.hip)
 template <typename T>
 int launchTriStage(fr_ctx *c, const frdev::StageArgs<T> &a, int mode);

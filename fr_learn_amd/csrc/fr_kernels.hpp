@@ -256,6 +256,7 @@ struct StageArgs {
   // disFn_fpts = Fn_fpts - disFn [ele][field][fpt]
   T *dbgF, *dbgFn, *dbgJ;
   int rev;  // walk each XCD's range of element blocks backwards (k_stage)
+  int fullTraces;  // write the traces of faces inside a block too (the adjoint reads them)
 };
 
 // Face f of the two faces normal to reference axis d (hex: x 2,3; y 4,5;
@@ -1199,7 +1200,7 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
   // updated state goes to sFd (free after (2)), so that sU keeps the stage
   // state other elements of the block read
   stageUpdate<D, P, NF, T, FIN, DEF, L>(a, s1, &sJ[slot][0][0], &sFd[slot][0][0], e, t, act, div, pb, pdet, pdt,
-                                        [&](int r) { return VIS || !(pnb[r] < 0 || inBlock(pnb[r])); });
+                                        [&](int r) { return VIS || !(pnb[r] < 0 || (inBlock(pnb[r]) && !a.fullTraces)); });
 }
 
 // The inviscid final-stage variant asks for 3 waves per SIMD (at most 168
