@@ -33,7 +33,8 @@ void freeAll(fr_ctx *c) {
                   c->adjLam,  c->adjOut,  c->adjNu,   c->adjW,    c->adjS[0], c->adjS[1],
                   c->adjS[2], c->adjS[3], c->adjB,    c->JGc64,  c->detJc, c->fgeoc64,
                   c->JGc32,   c->fgeoc32, c->waveSp,
-                  c->dtNum,   c->wsurf,   c->dtPart,  c->geoN64,  c->geoN32,  c->errTab, c->Xd};
+                  c->dtNum,   c->wsurf,   c->dtPart,  c->geoN64,  c->geoN32,  c->errTab, c->Xd,
+                  c->ipermD};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   for (auto &v : c->ev)
@@ -243,22 +244,49 @@ int updateOnce(fr_ctx *c) {
   return rc;
 }
 
-// reference layout [pt][ele][field] <-> device [device ele][field][pt]
-void refToDev(const fr_ctx *c, const double *src, double *dst, int NF, int NP) {
-  const int nE = c->nE;
-  for (int p = 0; p < NP; p++)
-    for (int e = 0; e < nE; e++) {
-      const size_t de = (size_t)c->iperm[e];
-      for (int k = 0; k < NF; k++) dst[(de * NF + k) * NP + p] = src[((size_t)p * nE + e) * NF + k];
-    }
+// Reference layout [pt][ele][field] of a host array <-> device
+// [device ele][field][pt], NP points per element.  The device changes the
+// layout (k_to_ref, k_from_ref); the reference-layout side passes through the
+// RK stage state Us, whose contents no call leaves for the next, in chunks of
+// points where it is smaller than the array.
+struct RefChunk {
+  int pts, et, lds;  // points per chunk, elements per workgroup, its LDS bytes
+};
+RefChunk refChunk(const fr_ctx *c, int NF, int NP) {
+  RefChunk r;
+  const size_t cap = c->nState() * c->tsize() / 8;
+  r.pts = (int)std::min<size_t>((size_t)NP, std::max<size_t>(1, cap / ((size_t)c->nE * NF)));
+  const int row = NF * (r.pts | 1) * 8;
+  r.et = std::max(1, std::min(16, 32768 / row));
+  r.lds = r.et * row;
+  return r;
 }
-void devToRef(const fr_ctx *c, const double *src, double *dst, int NF, int NP) {
-  const int nE = c->nE;
-  for (int p = 0; p < NP; p++)
-    for (int e = 0; e < nE; e++) {
-      const size_t de = (size_t)c->iperm[e];
-      for (int k = 0; k < NF; k++) dst[((size_t)p * nE + e) * NF + k] = src[(de * NF + k) * NP + p];
-    }
+int refToDev(fr_ctx *c, const double *src, double *dst, int NF, int NP) {
+  const RefChunk r = refChunk(c, NF, NP);
+  const size_t plane = (size_t)c->nE * NF;
+  for (int p = 0; p < NP; p += r.pts) {
+    const int np = std::min(r.pts, NP - p);
+    HIP_TRY(hipMemcpyAsync(c->Us, src + p * plane, np * plane * 8, hipMemcpyHostToDevice, c->stream));
+    hipLaunchKernelGGL(frdev::k_from_ref, dim3((c->nE + r.et - 1) / r.et), dim3(256), r.lds, c->stream,
+                       (const double *)c->Us, c->ipermD, NF, NP, c->nE, r.et, p, np, dst);
+    HIP_TRY(hipGetLastError());
+  }
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  return 0;
+}
+template <typename TD>
+int devToRef(fr_ctx *c, const TD *src, double *dst, int NF, int NP, double add = 0.0) {
+  const RefChunk r = refChunk(c, NF, NP);
+  const size_t plane = (size_t)c->nE * NF;
+  for (int p = 0; p < NP; p += r.pts) {
+    const int np = std::min(r.pts, NP - p);
+    hipLaunchKernelGGL(frdev::k_to_ref<TD>, dim3((c->nE + r.et - 1) / r.et), dim3(256), r.lds, c->stream, src,
+                       c->ipermD, NF, NP, c->nE, r.et, p, np, add, (double *)c->Us);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(dst + p * plane, c->Us, np * plane * 8, hipMemcpyDeviceToHost, c->stream));
+  }
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  return 0;
 }
 
 int syncU32(fr_ctx *c) {
@@ -618,6 +646,8 @@ int createImpl(const fr_config *cfg, const fr_mesh *m, int precision, fr_ctx *c)
     for (int i = 0; i < nE; i++) c->iperm[c->perm[i]] = i;
     for (int e = 0; e < nE; e++)
       if (c->iperm[e] < 0) return fail(FR_EMESH, "element order is not a permutation");
+    if ((rc = dmalloc(&c->ipermD, (size_t)nE))) return rc;
+    HIP_TRY(hipMemcpy(c->ipermD, c->iperm.data(), (size_t)nE * sizeof(int), hipMemcpyHostToDevice));
   }
   // geometry on device
   {
@@ -904,9 +934,7 @@ int fr_get_geometry(fr_ctx *c, int which, double *out) {
     for (int s = 0; s < NS; s++)
       for (int e = 0; e < nE; e++) out[(size_t)s * nE + e] = h[(size_t)c->iperm[e] * NS + s];
   } else if (which == 2) {
-    std::vector<double> h((size_t)nE * D * NFP);
-    HIP_TRY(hipMemcpy(h.data(), c->ownN, h.size() * 8, hipMemcpyDeviceToHost));
-    devToRef(c, h.data(), out, D, NFP);
+    return devToRef(c, (const double *)c->ownN, out, D, NFP);
   } else if (which == 3) {
     std::vector<double> h((size_t)nE * (D + 1) * NFP);
     HIP_TRY(hipMemcpy(h.data(), c->fgeo64, h.size() * 8, hipMemcpyDeviceToHost));
@@ -952,18 +980,13 @@ int fr_set_state(fr_ctx *c, const double *U, int layout) {
   if (layout != FR_LAYOUT_REF && layout != FR_LAYOUT_DEVICE) return fail(FR_EINVAL, "unknown layout");
   setEnergyOffset(c, U, layout);
   stateChanged(c);
+  int rc;
   if (layout == FR_LAYOUT_REF) {
-    std::vector<double> h(n);
-    refToDev(c, U, h.data(), c->NF, c->NS);
-    HIP_TRY(hipMemcpyAsync(c->U, h.data(), n * 8, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-  } else if (layout == FR_LAYOUT_DEVICE) {
-    HIP_TRY(hipMemcpyAsync(c->U, U, n * 8, hipMemcpyHostToDevice, c->stream));
+    if ((rc = refToDev(c, U, c->U, c->NF, c->NS))) return rc;
   } else {
-    return fail(FR_EINVAL, "unknown layout");
+    HIP_TRY(hipMemcpyAsync(c->U, U, n * 8, hipMemcpyHostToDevice, c->stream));
   }
-  int rc = syncU32(c);
-  if (rc) return rc;
+  if ((rc = syncU32(c))) return rc;
   c->traceOf = -1;
   HIP_TRY(hipStreamSynchronize(c->stream));
   return 0;
@@ -971,15 +994,9 @@ int fr_set_state(fr_ctx *c, const double *U, int layout) {
 
 int fr_get_state(fr_ctx *c, double *U, int layout) {
   if (!c || !U) return fail(FR_EINVAL, "null argument");
-  const size_t n = c->nState();
+  if (layout == FR_LAYOUT_REF) return devToRef(c, c->U, U, c->NF, c->NS);
   HIP_TRY(hipStreamSynchronize(c->stream));
-  if (layout == FR_LAYOUT_REF) {
-    std::vector<double> h(n);
-    HIP_TRY(hipMemcpy(h.data(), c->U, n * 8, hipMemcpyDeviceToHost));
-    devToRef(c, h.data(), U, c->NF, c->NS);
-  } else {
-    HIP_TRY(hipMemcpy(U, c->U, n * 8, hipMemcpyDeviceToHost));
-  }
+  HIP_TRY(hipMemcpy(U, c->U, c->nState() * 8, hipMemcpyDeviceToHost));
   return 0;
 }
 
@@ -993,18 +1010,18 @@ int fr_get_residual(fr_ctx *c, int step, double *out, int layout) {
   if (step < 0 || step >= c->nRK) return fail(FR_EINVAL, "step out of range");
   if (step == c->nRK - 1 && c->finalDropped)
     return fail(FR_EINVAL, "divF_spts of the final stage was not kept (fr_keep_final_residual)");
+  if (layout == FR_LAYOUT_REF)
+    return c->prec == FR_PREC_FP32 ? devToRef(c, (const float *)c->divF[step], out, c->NF, c->NS)
+                                   : devToRef(c, (const double *)c->divF[step], out, c->NF, c->NS);
   const size_t n = c->nState();
   HIP_TRY(hipStreamSynchronize(c->stream));
-  std::vector<double> h(n);
   if (c->prec == FR_PREC_FP32) {
     std::vector<float> f(n);
     HIP_TRY(hipMemcpy(f.data(), c->divF[step], n * 4, hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < n; i++) h[i] = f[i];
+    for (size_t i = 0; i < n; i++) out[i] = f[i];
   } else {
-    HIP_TRY(hipMemcpy(h.data(), c->divF[step], n * 8, hipMemcpyDeviceToHost));
+    HIP_TRY(hipMemcpy(out, c->divF[step], n * 8, hipMemcpyDeviceToHost));
   }
-  if (layout == FR_LAYOUT_REF) devToRef(c, h.data(), out, c->NF, c->NS);
-  else std::memcpy(out, h.data(), n * 8);
   return 0;
 }
 
@@ -1042,19 +1059,17 @@ int fr_get_array(fr_ctx *c, int which, double *out) {
     rc = launchStageDbg(c, a, dUf, dUs);
   }
   hipError_t err = hipStreamSynchronize(c->stream);
+  if (!rc && err == hipSuccess && (which == 3 || which == 4)) rc = devToRef(c, which == 3 ? dFn : dJ, out, NF, NFP);
   std::vector<double> h;
-  if (!rc && err == hipSuccess) {
-    const double *src = which == 2 ? dF : which == 3 ? dFn : which == 4 ? dJ : which == 5 ? dUs : dUf;
-    h.resize(which == 6 ? (size_t)nE * D * NF * NFP : (which == 2 || which == 5) ? nSp : nFp);
+  if (!rc && err == hipSuccess && which != 3 && which != 4) {
+    const double *src = which == 2 ? dF : which == 5 ? dUs : dUf;
+    h.resize(which == 6 ? (size_t)nE * D * NF * NFP : nSp);
     err = hipMemcpy(h.data(), src, h.size() * 8, hipMemcpyDeviceToHost);
   }
   release();
   if (rc) return rc;
   if (err != hipSuccess) return fail(FR_EHIP, std::string("fr_get_array: ") + hipGetErrorString(err));
-  if (which == 3 || which == 4) {
-    devToRef(c, h.data(), out, NF, NFP);
-    return 0;
-  }
+  if (which == 3 || which == 4) return 0;
   // (dim, point, ele, field) from the device's [ele][dim][field][point]
   const int NP = which == 6 ? NFP : NS;
   for (int d = 0; d < D; d++)
@@ -1069,25 +1084,14 @@ int fr_get_array(fr_ctx *c, int which, double *out) {
 
 int fr_get_traces(fr_ctx *c, double *out) {
   if (!c || !out) return fail(FR_EINVAL, "null argument");
-  const size_t n = (size_t)c->nE * c->NF * c->NFP;
   // the stage kernels exchange the traces of faces inside an element block
   // through LDS and leave them out of the trace buffer: extrapolate afresh
   c->traceOf = -1;
   int rc = (c->prec == FR_PREC_FP32) ? ensureTraces<float>(c, 0) : ensureTraces<double>(c, 0);
   if (rc) return rc;
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  std::vector<double> h(n);
-  if (c->prec == FR_PREC_FP32) {
-    std::vector<float> f(n);
-    HIP_TRY(hipMemcpy(f.data(), c->Uf[c->cur], n * 4, hipMemcpyDeviceToHost));
-    // the FP32 energy traces are offset (Phys::eOff)
-    for (size_t i = 0; i < n; i++)
-      h[i] = (double)f[i] + (((int)((i / c->NFP) % c->NF) == c->NF - 1) ? c->ph.eOff : 0.0);
-  } else {
-    HIP_TRY(hipMemcpy(h.data(), c->Uf[c->cur], n * 8, hipMemcpyDeviceToHost));
-  }
-  devToRef(c, h.data(), out, c->NF, c->NFP);
-  return 0;
+  // the FP32 energy traces are offset (Phys::eOff)
+  return c->prec == FR_PREC_FP32 ? devToRef(c, (const float *)c->Uf[c->cur], out, c->NF, c->NFP, c->ph.eOff)
+                                 : devToRef(c, (const double *)c->Uf[c->cur], out, c->NF, c->NFP);
 }
 
 int fr_update(fr_ctx *c, int nSteps) {
@@ -1241,15 +1245,9 @@ int fr_vjp_residual(fr_ctx *c, const double *lam, double *out) {
   if (!c || !lam || !out) return fail(FR_EINVAL, "null argument");
   int rc = adjCheck(c);
   if (rc) return rc;
-  const size_t n = c->nState();
-  std::vector<double> h(n);
-  refToDev(c, lam, h.data(), c->NF, c->NS);
-  HIP_TRY(hipMemcpyAsync(c->adjLam, h.data(), n * 8, hipMemcpyHostToDevice, c->stream));
+  if ((rc = refToDev(c, lam, c->adjLam, c->NF, c->NS))) return rc;
   if ((rc = vjpResidualDev(c, c->U, c->adjLam, c->adjOut))) return rc;
-  HIP_TRY(hipMemcpyAsync(h.data(), c->adjOut, n * 8, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  devToRef(c, h.data(), out, c->NF, c->NS);
-  return 0;
+  return devToRef(c, c->adjOut, out, c->NF, c->NS);
 }
 
 int fr_vjp_step(fr_ctx *c, const double *lam1, double *lam0) {
@@ -1259,15 +1257,9 @@ int fr_vjp_step(fr_ctx *c, const double *lam1, double *lam0) {
   // the step's time step is the one the next update takes (a constant of
   // the step); forming it here leaves it for that update
   if ((rc = dtPrepare(c, c->stream))) return rc;
-  const size_t n = c->nState();
-  std::vector<double> h(n);
-  refToDev(c, lam1, h.data(), c->NF, c->NS);
-  HIP_TRY(hipMemcpyAsync(c->adjLam, h.data(), n * 8, hipMemcpyHostToDevice, c->stream));
+  if ((rc = refToDev(c, lam1, c->adjLam, c->NF, c->NS))) return rc;
   if ((rc = vjpStepDev(c, c->adjLam, c->adjOut))) return rc;
-  HIP_TRY(hipMemcpyAsync(h.data(), c->adjOut, n * 8, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  devToRef(c, h.data(), lam0, c->NF, c->NS);
-  return 0;
+  return devToRef(c, c->adjOut, lam0, c->NF, c->NS);
 }
 
 int fr_vjp_steps(fr_ctx *c, int nSteps, int every, const double *lamN, double *lam0) {
@@ -1322,9 +1314,7 @@ int fr_vjp_steps(fr_ctx *c, int nSteps, int every, const double *lamN, double *l
   // reverse sweep, recomputing each segment's step states from its checkpoint
   // with the recorded time steps
   c->dtFrozen = cfl;
-  std::vector<double> h(n);
-  refToDev(c, lamN, h.data(), c->NF, c->NS);
-  HIP_TRY(hipMemcpyAsync(c->adjLam, h.data(), n * 8, hipMemcpyHostToDevice, c->stream));
+  if ((rc = refToDev(c, lamN, c->adjLam, c->NF, c->NS))) { cleanup(); return rc; }
   double *lamA = c->adjLam, *lamB = c->adjOut;
   for (int k = nCk - 1; k >= 0; k--) {
     const int start = k * every, end = std::min(start + every, nSteps);
@@ -1344,7 +1334,6 @@ int fr_vjp_steps(fr_ctx *c, int nSteps, int every, const double *lamN, double *l
       std::swap(lamA, lamB);
     }
   }
-  HIP_TRY(hipMemcpyAsync(h.data(), lamA, n * 8, hipMemcpyDeviceToHost, c->stream));
   if (copy(c->U, uN) != hipSuccess) { cleanup(); return fail(FR_EHIP, "copy"); }
   // the context as the forward sweep left it: the last step's time step and
   // the wave speeds of its last residual
@@ -1357,11 +1346,10 @@ int fr_vjp_steps(fr_ctx *c, int nSteps, int every, const double *lamN, double *l
     }
     c->dtReady = false;
   }
-  HIP_TRY(hipStreamSynchronize(c->stream));
   c->traceOf = -1;
+  rc = devToRef(c, lamA, lam0, c->NF, c->NS);
   cleanup();
-  devToRef(c, h.data(), lam0, c->NF, c->NS);
-  return syncU32(c);
+  return rc ? rc : syncU32(c);
 }
 
 int fr_reduce_gradient(fr_ctx *c, int kind, double *out) {
@@ -1379,14 +1367,11 @@ int fr_reduce_gradient(fr_ctx *c, int kind, double *out) {
   else
     hipLaunchKernelGGL(frdev::k_ke_grad<2>, dim3(nblk(nPts)), dim3(256), 0, c->stream, c->U, c->detJ, c->wts, c->NS,
                        nPts, g);
-  std::vector<double> h(n);
-  hipError_t e1 = hipGetLastError();
-  hipError_t e2 = hipMemcpyAsync(h.data(), g, n * 8, hipMemcpyDeviceToHost, c->stream);
-  hipError_t e3 = hipStreamSynchronize(c->stream);
+  const hipError_t e1 = hipGetLastError();
+  if (e1 == hipSuccess) rc = devToRef(c, g, out, c->NF, c->NS);
   (void)hipFree(g);
-  if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) return fail(FR_EHIP, "kinetic-energy gradient");
-  devToRef(c, h.data(), out, c->NF, c->NS);
-  return 0;
+  if (e1 != hipSuccess) return fail(FR_EHIP, "kinetic-energy gradient");
+  return rc;
 }
 
 #ifndef FR_BATCH_STREAMS

@@ -1364,6 +1364,49 @@ static __global__ void k_state_to_float(const double *__restrict__ U, float *__r
   if (i < n) U32[i] = stateToFloat(U[i], i, NF, NS, eOff);
 }
 
+// Layout changes at the ABI edge: the reference layout [pt][mesh ele][field]
+// of points p0 .. p0 + np of the mesh against the device's
+// [device ele][field][pt], mesh element e being device element iperm[e].  A
+// workgroup moves ET elements through LDS: the device side is one contiguous
+// block per element, the reference side a run of ET elements' fields per
+// point.  The copy to the host bounds a read-back (17 GB/s into pageable
+// memory): the 283 MB state of 48^3 P3 takes 27 ms with a fresh host array and
+// took 263 ms with the layout changed by a host loop, whose every access missed
+// the cache.  add (FP32 energies, Phys::eOff) goes to the last field.
+template <typename TD>
+__global__ __launch_bounds__(256) void k_to_ref(const TD *__restrict__ src, const int *__restrict__ iperm, int NF,
+                                                int NP, int nE, int ET, int p0, int np, double add,
+                                                double *__restrict__ ref) {
+  extern __shared__ double tile[];  // [ET][NF][np | 1]: an odd row stride
+  const int e0 = blockIdx.x * ET, ne = min(ET, nE - e0), st = np | 1;
+  for (int i = threadIdx.x; i < ne * NF * np; i += blockDim.x) {
+    const int r = i / np, p = i - r * np, e = r / NF, k = r - e * NF;
+    tile[r * st + p] = (double)src[((size_t)iperm[e0 + e] * NF + k) * NP + p0 + p] + (k == NF - 1 ? add : 0.0);
+  }
+  __syncthreads();
+  const int run = ne * NF;
+  for (int i = threadIdx.x; i < run * np; i += blockDim.x) {
+    const int p = i / run, r = i - p * run;
+    ref[((size_t)p * nE + e0) * NF + r] = tile[r * st + p];
+  }
+}
+static __global__ __launch_bounds__(256) void k_from_ref(const double *__restrict__ ref,
+                                                         const int *__restrict__ iperm, int NF, int NP, int nE, int ET,
+                                                         int p0, int np, double *__restrict__ dst) {
+  extern __shared__ double tile[];
+  const int e0 = blockIdx.x * ET, ne = min(ET, nE - e0), st = np | 1;
+  const int run = ne * NF;
+  for (int i = threadIdx.x; i < run * np; i += blockDim.x) {
+    const int p = i / run, r = i - p * run;
+    tile[r * st + p] = ref[((size_t)p * nE + e0) * NF + r];
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < run * np; i += blockDim.x) {
+    const int r = i / np, p = i - r * np, e = r / NF, k = r - e * NF;
+    dst[((size_t)iperm[e0 + e] * NF + k) * NP + p0 + p] = tile[r * st + p];
+  }
+}
+
 // CFL time step of each element from the current state, FP64: the traces
 // (extrapolateU), the wave speed |v.n| + c (Euler) or |a.n| (advection) at
 // every flux point (ele::calcWaveSpFpts, ele.cpp:1031-1084, static grids) and
