@@ -252,18 +252,71 @@ int updateOnce(fr_ctx *c) {
 struct RefChunk {
   int pts, et, lds;  // points per chunk, elements per workgroup, its LDS bytes
 };
-RefChunk refChunk(const fr_ctx *c, int NF, int NP) {
+RefChunk refChunk(const fr_ctx *c, int NF, int NP, int most) {
   RefChunk r;
-  const size_t cap = c->nState() * c->tsize() / 8;
-  r.pts = (int)std::min<size_t>((size_t)NP, std::max<size_t>(1, cap / ((size_t)c->nE * NF)));
+  r.pts = std::min(NP, most);
   const int row = NF * (r.pts | 1) * 8;
   r.et = std::max(1, std::min(16, 32768 / row));
   r.lds = r.et * row;
   return r;
 }
+// Points of all elements' NF fields that Us holds.
+int usPoints(const fr_ctx *c, int NF) {
+  return (int)std::max<size_t>(1, c->nState() * c->tsize() / 8 / ((size_t)c->nE * NF));
+}
+
+// Small arrays go through pinned host memory that the layout kernels access
+// themselves: one buffer for the process, made by the first of them and
+// freed with the last context.  A copy into the caller's pageable array costs the runtime
+// its pinning, most of all where the array is fresh, and a wait of its own
+// behind a busy stream: 74 KB 35 -> 6.5 us, 524 KB 60 -> 27 us, 40 arrays of
+// 0.65 MB 15 -> 9 ms fresh and 8.4 -> 4.3 ms reused.  From some MB on both move
+// 17 GB/s, so larger arrays are copied and the buffer stays small.  A thread that
+// finds the buffer in use takes the copy.
+constexpr size_t kStageBytes = 8u << 20;
+struct HostStage {
+  std::mutex m;
+  double *buf = nullptr;
+  int contexts = 0;
+};
+HostStage gStage;
+void stageRetain() {
+  std::lock_guard<std::mutex> lock(gStage.m);
+  gStage.contexts++;
+}
+void stageRelease() {
+  std::lock_guard<std::mutex> lock(gStage.m);
+  if (--gStage.contexts == 0 && gStage.buf) {
+    (void)hipHostFree(gStage.buf);
+    gStage.buf = nullptr;
+  }
+}
+
+// The buffer, held until the lock goes, or null: bytes too large, in use, or not
+// to be had.
+double *stageBuffer(std::unique_lock<std::mutex> &lock, size_t bytes) {
+  if (bytes > kStageBytes || !lock.try_lock()) return nullptr;
+  if (!gStage.buf &&
+      hipHostMalloc((void **)&gStage.buf, kStageBytes, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
+    gStage.buf = nullptr;
+    (void)hipGetLastError();
+  }
+  return gStage.buf;
+}
+
 int refToDev(fr_ctx *c, const double *src, double *dst, int NF, int NP) {
-  const RefChunk r = refChunk(c, NF, NP);
+  const RefChunk r = refChunk(c, NF, NP, usPoints(c, NF));
   const size_t plane = (size_t)c->nE * NF;
+  std::unique_lock<std::mutex> lock(gStage.m, std::defer_lock);
+  if (double *buf = stageBuffer(lock, plane * NP * 8)) {
+    const RefChunk w = refChunk(c, NF, NP, NP);
+    std::memcpy(buf, src, plane * NP * 8);
+    hipLaunchKernelGGL(frdev::k_from_ref, dim3((c->nE + w.et - 1) / w.et), dim3(256), w.lds, c->stream, buf,
+                       c->ipermD, NF, NP, c->nE, w.et, 0, NP, dst);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    return 0;
+  }
   for (int p = 0; p < NP; p += r.pts) {
     const int np = std::min(r.pts, NP - p);
     HIP_TRY(hipMemcpyAsync(c->Us, src + p * plane, np * plane * 8, hipMemcpyHostToDevice, c->stream));
@@ -276,8 +329,18 @@ int refToDev(fr_ctx *c, const double *src, double *dst, int NF, int NP) {
 }
 template <typename TD>
 int devToRef(fr_ctx *c, const TD *src, double *dst, int NF, int NP, double add = 0.0) {
-  const RefChunk r = refChunk(c, NF, NP);
+  const RefChunk r = refChunk(c, NF, NP, usPoints(c, NF));
   const size_t plane = (size_t)c->nE * NF;
+  std::unique_lock<std::mutex> lock(gStage.m, std::defer_lock);
+  if (double *buf = stageBuffer(lock, plane * NP * 8)) {
+    const RefChunk w = refChunk(c, NF, NP, NP);
+    hipLaunchKernelGGL(frdev::k_to_ref<TD>, dim3((c->nE + w.et - 1) / w.et), dim3(256), w.lds, c->stream, src,
+                       c->ipermD, NF, NP, c->nE, w.et, 0, NP, add, buf);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    std::memcpy(dst, buf, plane * NP * 8);
+    return 0;
+  }
   for (int p = 0; p < NP; p += r.pts) {
     const int np = std::min(r.pts, NP - p);
     hipLaunchKernelGGL(frdev::k_to_ref<TD>, dim3((c->nE + r.et - 1) / r.et), dim3(256), r.lds, c->stream, src,
@@ -876,6 +939,7 @@ int fr_create(const fr_config *cfg, const fr_mesh *mesh, int precision, fr_ctx *
     g_err = msg;
     return rc;
   }
+  stageRetain();
   *out = c;
   return 0;
 }
@@ -891,6 +955,7 @@ int fr_destroy(fr_ctx *c) {
   }
   freeAll(c);
   delete c;
+  stageRelease();
   return 0;
 }
 

@@ -1,6 +1,7 @@
-"""The layout changes at the ABI edge run on the device, through a scratch
-buffer of the stage state's size and in chunks of points where that is smaller
-than the array (FP32 contexts, traces).  Sizes at the edges: element counts
+"""The layout changes at the ABI edge run on the device: arrays of up to 8 MB
+into a pinned host buffer, larger ones through a scratch buffer of the stage
+state's size, in chunks of points where that is smaller than the array (FP32
+contexts, traces).  Sizes at the edges: element counts
 that are no multiple of a workgroup's elements, one field, the smallest and
 largest elements."""
 import numpy as np
@@ -11,7 +12,7 @@ from fr_learn_amd import Solver, _lib, cases, mesh
 pytestmark = pytest.mark.gpu
 
 SHAPES = [("quad", 1, (3, 3)), ("quad", 4, (7, 5)), ("quad", 5, (41, 3)), ("tri", 2, (5, 4)), ("tri", 5, (3, 7)),
-          ("hex", 1, (3, 4, 5)), ("hex", 3, (3, 3, 4)), ("hex", 5, (3, 3, 3))]
+          ("quad", 5, (103, 101)), ("hex", 1, (3, 4, 5)), ("hex", 3, (3, 3, 4)), ("hex", 5, (3, 3, 3)), ("hex", 3, (17, 16, 19))]
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
@@ -45,3 +46,32 @@ def test_state_layouts(elem, P, n, equation, precision):
     tol = 1e-13 if precision == "fp64" else 2e-6
     assert np.abs(g.traces() - want).max() <= tol * np.abs(want).max()
     g.close()
+
+
+def test_read_backs_from_several_threads():
+    """The pinned buffer is one for the process: threads that meet at it get
+    their own context's state."""
+    import threading
+    solvers, states = [], []
+    for i in range(4):
+        cfg = cases.config(nDims=2, order=3)
+        s = Solver(cfg, mesh.box(2, (9 + i, 40), (0.0, 0.0), (1.0, 1.0)))
+        U = np.random.default_rng(i).uniform(1.0, 2.0, s.state_shape())
+        s.set_state(U)
+        solvers.append(s)
+        states.append(U)
+    wrong = []
+
+    def work(i):
+        for _ in range(200):
+            if not np.array_equal(solvers[i].get_state(), states[i]):
+                wrong.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    for s in solvers:
+        s.close()
