@@ -696,7 +696,10 @@ int createImpl(const fr_config *cfg, const fr_mesh *m, int precision, fr_ctx *c)
   }
   // device element order: blocks of EPB face-connected elements
   dispatch(D, c->P, c->NF, [&](auto Dc, auto Pc, auto) {
-    c->epb = frdev::ElemGeo<decltype(Dc)::value, decltype(Pc)::value>::EPB;
+    constexpr int D = decltype(Dc)::value, P = decltype(Pc)::value;
+    c->epb = frdev::ElemGeo<D, P>::EPB;
+    if constexpr (frdev::packedOrder(D, P))
+      if (!cfg->viscous && frdev::stageTile(D, P, c->nE)) c->epb = frdev::ElemGeo<D, P, 1>::EPB;
   });
   if (c->tri) c->epb = 256 / frdev::triTPE(c->P);  // frdev::TriGeo<P>::EPB
   {

@@ -246,6 +246,7 @@ struct StageArgs {
   double *waveSp;             // CFL wave speeds [ele][fpt] written at left / boundary points, or null
   double c0, c1, c2, c3, rk;
   int mode, nprev, nEles;
+  int fullTraces;  // write the traces of faces inside a block too (the adjoint reads them)
   Phys ph;
   int affine;  // geometry layout (GeoAddr)
   int nodal;   // 1: the stage kernel forms its metrics and normals from geoN (GM = 1)
@@ -256,7 +257,6 @@ struct StageArgs {
   // disFn_fpts = Fn_fpts - disFn [ele][field][fpt]
   T *dbgF, *dbgFn, *dbgJ;
   int rev;  // walk each XCD's range of element blocks backwards (k_stage)
-  int fullTraces;  // write the traces of faces inside a block too (the adjoint reads them)
 };
 
 // Face f of the two faces normal to reference axis d (hex: x 2,3; y 4,5;
@@ -757,12 +757,13 @@ __device__ __forceinline__ void subtractEarlier(const StageArgs<T> &a, const T (
 // area-weighted normal, whose length is dA; a right-side point uses the
 // negated own normal for the left element's (equal but for rounding).
 // GM = 2 forms the solution-point metrics and reads the face geometry.
-// L is the tile layout (ElemGeo): 1 only in the batched 2D kernels.
+// L is the tile layout (ElemGeo): 1 in the batched 2D kernels and for P5 quads
+// (stageTile).
 template <int D, int P, int NF, typename T, bool BND, bool VIS, bool FIN, int GM = 0, bool DBG = false, int L = 0>
 __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, StageSmem<D, P, NF, T, L> &sm,
                                           const int tid) {
   static_assert(GM == 0 || !VIS, "the viscous stage reads the per-point geometry");
-  static_assert(L == 0 || (D == 2 && !VIS), "layout 1 is the inviscid 2D batch layout");
+  static_assert(L == 0 || (D == 2 && !VIS), "layout 1 is an inviscid 2D layout");
   using G = ElemGeo<D, P, L>;
   using O = OneD<P>;
   constexpr int NS = G::NS, NFP = G::NFP, NFPF = G::NFPF, P1 = G::P1, TPE = G::TPE, EPB = G::EPB;
@@ -1207,12 +1208,12 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
 // VGPRs): it holds the most prefetched data, and at 2 waves per SIMD the
 // final stage ran 12 % longer.  So do the hex P3 variants with the MFMA
 // contractions, whose accumulators would otherwise take them to 2 waves.
-template <int D, int P, int NF, typename T, bool BND, bool FIN, int GM = 0>
-__global__ __launch_bounds__((ElemGeo<D, P>::NTH),
+template <int D, int P, int NF, typename T, bool BND, bool FIN, int GM = 0, int L = 0>
+__global__ __launch_bounds__((ElemGeo<D, P, L>::NTH),
                              ((FR_MFMA && D == 3 && P == 3) ? (FIN ? FR_MF_FIN_WAVES : FR_MF_WAVES)
                               : FIN                          ? 3
                                                              : FR_STAGE_MINW)) void k_stage(StageArgs<T> a) {
-  __shared__ StageSmem<D, P, NF, T> sm;
+  __shared__ StageSmem<D, P, NF, T, L> sm;
   // Workgroups are dealt to the 8 XCDs in turn; remap so that each XCD walks a
   // contiguous range of elements and face neighbours share its L2.  The host
   // pads the grid to a multiple of 8.  rev walks the range backwards, so that
@@ -1220,7 +1221,7 @@ __global__ __launch_bounds__((ElemGeo<D, P>::NTH),
   // in the memory-side cache).
   const int R = gridDim.x >> 3, j = blockIdx.x >> 3;
   const int b = (blockIdx.x & 7) * R + (a.rev ? R - 1 - j : j);
-  stageBody<D, P, NF, T, BND, false, FIN, GM>(a, b, sm, (int)threadIdx.x);
+  stageBody<D, P, NF, T, BND, false, FIN, GM, false, L>(a, b, sm, (int)threadIdx.x);
 }
 
 // The residual evaluation (mode 0) with the debug outputs of StageArgs

@@ -53,6 +53,16 @@ constexpr int tensorTPE(int D, int P, int L) {
   return nextPow2(ns) < 8 ? 8 : nextPow2(ns);
 }
 
+// Tile layout of the per-mesh inviscid stage kernels: the packed one for P5
+// quads from 4096 elements on, where 36 of layout 0's 64 threads per element
+// hold a point and the chip is full (us a stage, Roe: 128^2 FP64 36.0 -> 27.8,
+// FP32 23.8 -> 20.8; 64^2 FP64 11.9 -> 11.0, FP32 8.9 -> 8.9).  Its phases need
+// workgroup barriers, which smaller meshes feel (24^2 FP64 6.4 -> 6.7) and which
+// cost the other orders more than their lanes gain (Rusanov, 128^2 FP64: P2
+// 10.4 -> 12.0, P4 20.1 -> 20.5).
+constexpr bool packedOrder(int D, int P) { return D == 2 && P == 5; }
+constexpr int stageTile(int D, int P, int nEles) { return packedOrder(D, P) && nEles >= 4096 ? 1 : 0; }
+
 template <int D, int P, int L = 0>
 struct ElemGeo {
   static constexpr int P1 = P + 1;

@@ -23,9 +23,9 @@ int launchStageArgsD(fr_ctx *c, const frdev::StageArgs<T> &a, int mode) {
       return;
     } else {
     using G = frdev::ElemGeo<D, P>;
-    // grid padded to a multiple of the 8 XCDs (the kernels remap block ids)
-    const unsigned nb = (unsigned)(((c->nE + G::EPB - 1) / G::EPB + 7) / 8 * 8);
+    // grids padded to a multiple of the 8 XCDs (the kernels remap block ids)
     if (vis) {
+      const unsigned nb = (unsigned)(((c->nE + G::EPB - 1) / G::EPB + 7) / 8 * 8);
       {
         TimeScope ts(c, 3);
         if (bnd) hipLaunchKernelGGL((frdev::k_visc_flux<D, P, NF, T, true>), dim3(nb), dim3(G::NTH), 0, c->stream, a,
@@ -47,10 +47,22 @@ int launchStageArgsD(fr_ctx *c, const frdev::StageArgs<T> &a, int mode) {
       TimeScope ts(c, 0);
       // the inviscid variants: boundary faces or not, final stage or not,
       // geometry from the stored arrays or from the nodal map (GM)
-      auto launch = [&](auto Bc, auto Fc, auto Gc) {
+      auto launchL = [&](auto Bc, auto Fc, auto Gc, auto Lc) {
+        constexpr int L = decltype(Lc)::value;
+        using GL = frdev::ElemGeo<D, P, L>;
+        const unsigned n = (unsigned)(((c->nE + GL::EPB - 1) / GL::EPB + 7) / 8 * 8);
         hipLaunchKernelGGL((frdev::k_stage<D, P, NF, T, decltype(Bc)::value, decltype(Fc)::value,
-                                           decltype(Gc)::value>),
-                           dim3(nb), dim3(G::NTH), 0, c->stream, a);
+                                           decltype(Gc)::value, L>),
+                           dim3(n), dim3(GL::NTH), 0, c->stream, a);
+      };
+      auto launch = [&](auto Bc, auto Fc, auto Gc) {
+        if constexpr (frdev::packedOrder(D, P)) {
+          if (frdev::stageTile(D, P, c->nE)) {
+            launchL(Bc, Fc, Gc, std::integral_constant<int, 1>{});
+            return;
+          }
+        }
+        launchL(Bc, Fc, Gc, std::integral_constant<int, 0>{});
       };
       auto byGeo = [&](auto Bc, auto Fc) {
         if (a.nodal == 1) launch(Bc, Fc, std::integral_constant<int, 1>{});
