@@ -862,7 +862,8 @@ int createImpl(const fr_config *cfg, const fr_mesh *m, int precision, fr_ctx *c)
 // Buffers of CFL time stepping (allocated by the first fr_calc_dt).
 int cflBuffers(fr_ctx *c) {
   int rc;
-  const size_t nb = nblk(c->nE);
+  // block minima: of workgroups of as few as 4 elements (k_dt_ws, 64 lanes each)
+  const size_t nb = nblk(c->nE, 4);
   if ((!c->dtE && (rc = dmalloc(&c->dtE, (size_t)c->nE))) ||
       (!c->waveSp && (rc = dmalloc(&c->waveSp, (size_t)c->nE * c->NFP))) ||
       (!c->dtNum && (rc = dmalloc(&c->dtNum, (size_t)c->nE))) || (!c->dtPart && (rc = dmalloc(&c->dtPart, nb))))
@@ -893,32 +894,34 @@ int dtPrepare(fr_ctx *c, hipStream_t st) {
   // getCFLLimit (global.cpp:45-68)
   static const double lim[6] = {1.393, 0.464, 0.235, 0.1453, 0.100, 0.0736};
   const double factor = c->cfl * lim[c->P] * 2;
-  const unsigned nb = nblk(c->nE);
+  unsigned nPart = 0;  // workgroup minima
   hipError_t err = hipSuccess;
   if (c->tri) {
     // triangles (no reference counterpart): the wave speeds of the current
     // state at every update
     int rc = launchTriDt(c, c->wsurf, factor, st);
     if (rc) return rc;
-    hipLaunchKernelGGL(frdev::k_block_min, dim3(nb), dim3(256), 0, st, c->dtE, c->nE, c->dtPart);
+    nPart = nblk(c->nE, 256 / frdev::triTPE(c->P));
   } else if (c->dtFirst) {
     // the first update: ele::calcWaveSpFpts from the state (solver.cpp:294-297)
+    nPart = nblk(c->nE);
     dispatch(c->D, c->P, c->NF, [&](auto Dc, auto Pc, auto NFc) {
       constexpr int D = decltype(Dc)::value, P = decltype(Pc)::value, NF = decltype(NFc)::value;
-      hipLaunchKernelGGL((frdev::k_dt<D, P, NF>), dim3(nb), dim3(256), 0, st, c->U, c->ownN, c->fgeo64, c->detJ,
+      hipLaunchKernelGGL((frdev::k_dt<D, P, NF>), dim3(nPart), dim3(256), 0, st, c->U, c->ownN, c->fgeo64, c->detJ,
                          c->wts, c->wsurf, c->oned64, factor, c->ph, c->nE, c->dtE, c->waveSp, c->dtNum);
     });
     if ((err = hipGetLastError()) != hipSuccess) return fail(FR_EHIP, std::string("k_dt: ") + hipGetErrorString(err));
-    hipLaunchKernelGGL(frdev::k_block_min, dim3(nb), dim3(256), 0, st, c->dtE, c->nE, c->dtPart);
+    hipLaunchKernelGGL(frdev::k_block_min, dim3(nPart), dim3(256), 0, st, c->dtE, c->nE, c->dtPart);
   } else {
     // later updates: the wave speeds the last residual's face fluxes stored
     dispatch(c->D, c->P, c->NF, [&](auto Dc, auto Pc, auto) {
       using G = frdev::ElemGeo<decltype(Dc)::value, decltype(Pc)::value>;
-      hipLaunchKernelGGL((frdev::k_dt_ws<G::NFP, G::NFPF>), dim3(nb), dim3(256), 0, st, c->waveSp, c->fgeo64,
+      nPart = nblk(c->nE, 256 / frdev::dtLanes(G::NFP));
+      hipLaunchKernelGGL((frdev::k_dt_ws<G::NFP, G::NFPF>), dim3(nPart), dim3(256), 0, st, c->waveSp, c->fgeo64,
                          c->wsurf, c->dtNum, c->D, c->nE, c->dtE, c->dtPart);
     });
   }
-  hipLaunchKernelGGL(frdev::k_dt_min, dim3(1), dim3(256), 0, st, c->dtPart, (int)nb, c->dtG);
+  hipLaunchKernelGGL(frdev::k_dt_min, dim3(1), dim3(nPart > 256 ? 1024 : 256), 0, st, c->dtPart, (int)nPart, c->dtG);
   if ((err = hipGetLastError()) != hipSuccess) return fail(FR_EHIP, std::string("time step: ") + hipGetErrorString(err));
   c->dtReady = true;
   return 0;

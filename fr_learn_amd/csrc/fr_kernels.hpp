@@ -1464,26 +1464,11 @@ __global__ __launch_bounds__(256) void k_dt(const double *__restrict__ U, const 
   dtNum[e] = factor * vol;
 }
 
-// The CFL time step of every element from the stored wave speeds
-// (ele::calcDt, ele.cpp:1086-1105, with the waveSp_fpts the face fluxes of
-// the last residual left: solver::calcDt after the first iteration,
-// solver.cpp:293-305), and the minimum over each block of elements into
-// part[block].  One thread per element.
-template <int NFP, int NFPF>
-__global__ __launch_bounds__(256) void k_dt_ws(const double *__restrict__ waveSp, const double *__restrict__ fgeo,
-                                               const double *__restrict__ wsurf, const double *__restrict__ dtNum,
-                                               int D, int nEles, double *__restrict__ dtE, double *__restrict__ part) {
-  __shared__ double red[256];
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  double dt = INFINITY;
-  if (e < nEles) {
-    const double *ws = waveSp + (size_t)e * NFP;
-    const double *dA = fgeo + ((size_t)e * (D + 1) + D) * NFP;
-    double intWave = 0;
-    for (int q = 0; q < NFP; q++) intWave += ws[q] * wsurf[q % NFPF] * dA[q];
-    dt = dtNum[e] / intWave;
-    dtE[e] = dt;
-  }
+// part[block] = the minimum of dt over the workgroup of 256 threads.  k_dt_min
+// finishes it in a launch of its own: a last workgroup found by an atomic
+// ticket instead made the CFL step of 7526 triangles 15 us against 8.5 (every
+// workgroup's ticket goes to one address beyond the XCDs' L2).
+__device__ __forceinline__ void blockMin(double dt, double *red, double *part) {
   red[threadIdx.x] = dt;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
@@ -1493,33 +1478,62 @@ __global__ __launch_bounds__(256) void k_dt_ws(const double *__restrict__ waveSp
   if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
+// Sum over the LPE lanes of a group (a power of two inside one wavefront).
+template <int LPE>
+__device__ __forceinline__ double groupSum(double x) {
+#pragma unroll
+  for (int m = 1; m < LPE; m <<= 1) x += __shfl_xor(x, m);
+  return x;
+}
+
+// The CFL time step of every element from the stored wave speeds
+// (ele::calcDt, ele.cpp:1086-1105, with the waveSp_fpts the face fluxes of
+// the last residual left: solver::calcDt after the first iteration,
+// solver.cpp:293-305), and each workgroup's minimum in part.  dtLanes lanes per
+// element, so that its flux points are read side by side (one thread per element
+// before, with a stride of the element between neighbouring lanes).
+constexpr int dtLanes(int NFP) { return NFP <= 16 ? 16 : NFP <= 64 ? 32 : 64; }
+
+template <int NFP, int NFPF>
+__global__ __launch_bounds__(256) void k_dt_ws(const double *__restrict__ waveSp, const double *__restrict__ fgeo,
+                                               const double *__restrict__ wsurf, const double *__restrict__ dtNum,
+                                               int D, int nEles, double *__restrict__ dtE, double *__restrict__ part) {
+  constexpr int LPE = dtLanes(NFP);
+  __shared__ double red[256];
+  const int e = blockIdx.x * (256 / LPE) + threadIdx.x / LPE, l = threadIdx.x % LPE;
+  const size_t ec = (size_t)min(e, nEles - 1);
+  const double *ws = waveSp + ec * NFP;
+  const double *dA = fgeo + (ec * (D + 1) + D) * NFP;
+  double intWave = 0;
+  for (int q = l; q < NFP; q += LPE) intWave += ws[q] * wsurf[q % NFPF] * dA[q];
+  intWave = groupSum<LPE>(intWave);
+  const double dt = dtNum[ec] / intWave;
+  if (l == 0 && e < nEles) dtE[e] = dt;
+  blockMin(e < nEles ? dt : INFINITY, red, part);
+}
+
 // part[block] = the minimum of x over each block of 256 entries.
 static __global__ __launch_bounds__(256) void k_block_min(const double *__restrict__ x, int n,
                                                           double *__restrict__ part) {
   __shared__ double red[256];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  red[threadIdx.x] = i < n ? x[i] : INFINITY;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] = fmin(red[threadIdx.x], red[threadIdx.x + w]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+  blockMin(i < n ? x[i] : INFINITY, red, part);
 }
 
 // dtG[0] = the minimum of part[0..n) (params->dt of solver::calcDt), one block.
-static __global__ __launch_bounds__(256) void k_dt_min(const double *__restrict__ part, int n,
-                                                       double *__restrict__ dtG) {
-  __shared__ double red[256];
+static __global__ __launch_bounds__(1024) void k_dt_min(const double *__restrict__ part, int n,
+                                                        double *__restrict__ dtG) {
+  __shared__ double red[16];
   double m = INFINITY;
   for (int i = threadIdx.x; i < n; i += blockDim.x) m = fmin(m, part[i]);
-  red[threadIdx.x] = m;
+#pragma unroll
+  for (int w = 1; w < 64; w <<= 1) m = fmin(m, __shfl_xor(m, w));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] = fmin(red[threadIdx.x], red[threadIdx.x + w]);
-    __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < (int)(blockDim.x >> 6); w++) m = fmin(m, red[w]);
+    dtG[0] = m;
   }
-  if (threadIdx.x == 0) dtG[0] = red[0];
 }
 
 // Affine-element test and compact geometry (GeoAddr): element e passes when
