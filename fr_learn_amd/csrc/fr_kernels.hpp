@@ -628,101 +628,27 @@ __device__ __forceinline__ void correctedGradient(const T *s1, const T *sUe, con
 template <int D, int P, int NF, typename T, int L = 0>
 struct StageSmem {
   using G = ElemGeo<D, P, L>;
+  // The contravariant fluxes of all axes are staged at once, so that the line
+  // sums of every axis follow one synchronisation: one array per axis, the first
+  // later the updated state's.  Hexes, whose workgroups per CU the LDS would
+  // otherwise cost, put the last axis where the jump goes afterwards if it fits.
+  // Hex P3 keeps them in registers (matrix cores).  These meshes wait on the
+  // chain of LDS phases, not on bytes: with one synchronisation for two an axis,
+  // P5 hexes (17 x 15 x 13, FP64, 200 steps of RK4) took 37.7 -> 35.4 ms, 40 mixed
+  // small meshes in one graph 28.4 -> 26.9, P4 quads (128^2) 38.9 -> 38.5.
+  static constexpr bool MF = FR_MFMA && D == 3 && P == 3;
+  static constexpr bool SHARE = !MF && D == 3 && G::NFP >= G::NSP;
+  static constexpr int NX = MF ? 0 : D - 1 - (SHARE ? 1 : 0);
   T sU[G::EPB][NF][G::NSP];   // stage state (padded rows, padIdx)
-  T sFd[G::EPB][NF][G::NSP];  // contravariant flux F~_d of one reference axis, later the updated state
+  T sFd[G::EPB][NF][G::NSP];  // contravariant flux F~_0, later the updated state
   T sJ[G::EPB][NF][G::NFP];   // normal-flux jump Fn*dA - disFn at the flux points
   T s1[OneD<P>::SIZE];        // 1D factor table
+  T sFx[NX ? NX : 1][NX ? G::EPB : 1][NX ? NF : 1][NX ? G::NSP : 1];  // F~_1 and, unless shared, F~_2
+  // F~_d of element slot, [NF][NSP]
+  __device__ __forceinline__ T *axis(int d, int slot) {
+    return d == 0 ? &sFd[slot][0][0] : SHARE && d == D - 1 ? &sJ[slot][0][0] : &sFx[d - 1][slot][0][0];
+  }
 };
-
-// The end of a stage, phases (4) and (5) of stageBody: the correction of the
-// jumps sJe [NF][NFP] (correctDivFlux, solver.cpp:789-806) added to the
-// divergence div, the stage update from the base pb (final stages: with the
-// earlier residuals' terms already subtracted), and the face traces of the
-// updated state, staged in sSe [NF][NSP].  face(r) is false for the rounds
-// whose flux point needs no trace in HBM.
-template <int D, int P, int NF, typename T, bool FIN, bool DEF, int L, typename Face>
-__device__ __forceinline__ void stageUpdate(const StageArgs<T> &a, const T *s1, const T *sJe, T *sSe, const int e,
-                                            const int t, const bool act, const T *div, const double *pb,
-                                            const double pdet, const double pdt, Face face) {
-  using G = ElemGeo<D, P, L>;
-  using O = OneD<P>;
-  constexpr int NS = G::NS, NSP = G::NSP, NFP = G::NFP, P1 = G::P1, TPE = G::TPE, NFACE = G::NFACE;
-  constexpr int NQ = (NFP + TPE - 1) / TPE;
-  constexpr bool MF = FR_MFMA && D == 3 && P == 3, MFF = MF && sizeof(T) == 8;
-  // the FP64 base of the final stages is absolute; FP32 stage states hold the
-  // energy less Phys::eOff
-  constexpr bool base64 = FIN;
-  T utv[NF];  // the updated state at this thread's point
-  if (act && t < NS) {
-    int cq[NFACE], cside[NFACE], cax[NFACE];
-    corrEntries<D, P>(t, cq, cside, cax);
-    T cw[NFACE];  // correction weights, read once for all fields
-#pragma unroll
-    for (int f = 0; f < NFACE; f++) cw[f] = s1[(cside[f] ? O::GR : O::GL) + cax[f]];
-    const size_t eo = (size_t)e * NF * NS;
-#pragma unroll
-    for (int k = 0; k < NF; k++) {
-      T corr = (T)0;
-#pragma unroll
-      for (int f = 0; f < NFACE; f++) corr += cw[f] * sJe[k * NFP + cq[f]];
-      const T dv = corr + div[k];
-      const size_t gi = eo + (size_t)k * NS + t;
-      if (a.divF) __builtin_nontemporal_store(dv, a.divF + gi);
-      if (!FIN && a.mode == 0) continue;
-      // stage terms RK * divF / detJ * dt, with dt / detJ formed once per point
-      const double dtJ = pdt / pdet;
-      double u = pb[k];
-      // DEF: the base state read again here instead of kept in registers
-      if constexpr (DEF) u = (double)a.UbaseT[gi];
-      if (FIN && a.mode == 2) {
-        // earlier residuals: already subtracted from pb
-        const double cl = (a.nprev == 0) ? a.c0 : (a.nprev == 1) ? a.c1 : (a.nprev == 2) ? a.c2 : a.c3;
-        u -= cl * (double)dv * dtJ;
-      } else {
-        u = u - a.rk * (double)dv * dtJ;
-      }
-      // the updated state in the residual precision, for the traces
-      double ut = u;
-      if constexpr (hasEnergyOffset<T>())
-        if (k == NF - 1 && base64) ut = u - a.ph.eOff;
-      if constexpr (!FIN) {
-        if (a.Unext) __builtin_nontemporal_store((T)u, a.Unext + gi);
-      } else {
-        __builtin_nontemporal_store(u, a.Uout + gi);
-        if (a.Uout32) __builtin_nontemporal_store((float)ut, a.Uout32 + gi);
-      }
-      sSe[k * NSP + padIdx<P>(t)] = (T)ut;
-      utv[k] = (T)ut;
-    }
-  }
-  if (!FIN && a.mode == 0) return;
-  elementSync<TPE>();
-  if (!act) return;
-  T *Fe = a.UfOut + (size_t)e * NF * NFP;
-#pragma unroll
-  for (int r = 0; r < NQ; r++) {
-    const int q = MF ? mfmaFpt(t, r) : t + r * TPE;
-    T tv[NF];
-    if constexpr (MFF) mfmaFaceRound<NF, NSP, T>(s1, sSe, t, utv, r, tv);
-    if (q >= NFP || !face(r)) continue;
-    if constexpr (MFF) {
-#pragma unroll
-      for (int k = 0; k < NF; k++) __builtin_nontemporal_store(tv[k], Fe + k * NFP + q);
-      continue;
-    }
-    int base, stride, side, dn;
-    fptLine<D, P>(q, base, stride, side, dn);
-    const int lb = padIdx<P>(base), ls = padStride<P>(stride);
-    const T *l1 = s1 + (side ? O::LR : O::LL);
-#pragma unroll
-    for (int k = 0; k < NF; k++) {
-      T acc = (T)0;
-#pragma unroll
-      for (int m = 0; m < P1; m++) acc += l1[m] * sSe[k * NSP + lb + m * ls];
-      __builtin_nontemporal_store(acc, Fe + k * NFP + q);
-    }
-  }
-}
 
 // The earlier residuals' terms of the final update (mode 2), subtracted from
 // the base in stage order as the timeStepB passes do.
@@ -795,7 +721,7 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
   // Faces between two elements of this block take the neighbour's trace from
   // its state in LDS (line sums), and their traces are not written to HBM (the
   // element order groups face neighbours into blocks).  The viscous variant
-  // keeps the full trace exchange, which k_grad reads, and so does the FP32
+  // (the debug instance) keeps the full trace exchange, and so does the FP32
   // matrix-core variant (hex P3 FP32 31.97 against 30.38 GDOF/s with it; the
   // FP64 one gains, 20.47 -> 21.02, since its step is bound by its bytes).
   const int blockBase = b * EPB;
@@ -1019,17 +945,52 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
         for (int k = 0; k < NF; k++) F[d][k] = Fv[d][k] + F[d][k];
     }
   }
-  // (2) per reference axis d: F~_d = sum_d2 JGinv(d,d2) F_d2, its derivative
-  // along d (calcDivF_spts) and its extrapolation to the two faces normal to d
-  // (extrapolateNormalFlux), stored negated as the start of the jump
+  // (2) F~_d = sum_d2 JGinv(d,d2) F_d2 of every reference axis d, and the sum of
+  // their derivatives along d (calcDivF_spts) with the correction of the
+  // extrapolated flux folded in
   if constexpr (MF) {
     if constexpr (FOLD) {
       if (act) mfmaDivergence<NF, T>(s1, t, pJ, F, div);
-      elementSync<TPE>();
     } else {
       if (act) mfmaAxes<NF, T>(sm, slot, t, pJ, F, div, a.dbgF + (size_t)e * D * NF * NS);
     }
+  } else if constexpr (FOLD) {
+    constexpr int NSP = G::NSP;
+    if (hasS)
+#pragma unroll
+      for (int d = 0; d < D; d++) {
+        T *x = sm.axis(d, slot);
+#pragma unroll
+        for (int k = 0; k < NF; k++) {
+          T acc = (T)0;
+#pragma unroll
+          for (int d2 = 0; d2 < D; d2++) acc += pJ[d * D + d2] * F[d2][k];
+          x[k * NSP + tP] = acc;
+        }
+      }
+    elementSync<TPE>();
+    if (hasS)
+#pragma unroll
+      for (int d = 0; d < D; d++) {
+        const T *x = sm.axis(d, slot);
+        const int id = (d == 0) ? si : (d == 1) ? sj : sk;
+#pragma unroll
+        for (int k = 0; k < NF; k++) {
+          T acc = (T)0;
+#pragma unroll
+          for (int m = 0; m < P1; m++) {
+            // LDS index of the line point
+            const int sp = padIdx<P>((d == 0)   ? m + P1 * (sj + P1 * sk)
+                                     : (d == 1) ? si + P1 * (m + P1 * sk)
+                                                : si + P1 * (sj + P1 * m));
+            acc += s1[O::DMF + id * P1 + m] * x[k * NSP + sp];
+          }
+          div[k] = (d == 0) ? acc : acc + div[k];
+        }
+      }
+    if constexpr (StageSmem<D, P, NF, T, L>::SHARE) elementSync<TPE>();  // the jump takes the last axis' place
   } else {
+    // the debug instance: axis by axis, with the face values of F~
 #pragma unroll
     for (int d = 0; d < D; d++) {
       if (hasS) {
@@ -1039,7 +1000,7 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
 #pragma unroll
           for (int d2 = 0; d2 < D; d2++) acc += pJ[d * D + d2] * F[d2][k];
           sFd[slot][k][tP] = acc;
-          if constexpr (DBG) a.dbgF[(((size_t)e * D + d) * NF + k) * NS + t] = acc;
+          a.dbgF[(((size_t)e * D + d) * NF + k) * NS + t] = acc;
         }
       }
       elementSync<TPE>();
@@ -1054,12 +1015,12 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
             const int sp = padIdx<P>((d == 0) ? m + P1 * (sj + P1 * sk)
                                      : (d == 1) ? si + P1 * (m + P1 * sk)
                                                 : si + P1 * (sj + P1 * m));
-            acc += s1[(FOLD ? O::DMF : O::DM) + id * P1 + m] * sFd[slot][k][sp];
+            acc += s1[O::DM + id * P1 + m] * sFd[slot][k][sp];
           }
           div[k] = (d == 0) ? acc : acc + div[k];
         }
       }
-      if (!FOLD && act && t < 2 * NFPF) {
+      if (act && t < 2 * NFPF) {
         const int q = dirFace<D>(d, t / NFPF) * NFPF + t % NFPF;
         int base, stride, side, dn;
         fptLine<D, P>(q, base, stride, side, dn);
@@ -1196,12 +1157,90 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
   }
   elementSync<TPE>();
 
-  // (4) correction of the jump and the stage update, (5) the traces of the
-  // updated state for the faces whose neighbour is in another block; the
-  // updated state goes to sFd (free after (2)), so that sU keeps the stage
-  // state other elements of the block read
-  stageUpdate<D, P, NF, T, FIN, DEF, L>(a, s1, &sJ[slot][0][0], &sFd[slot][0][0], e, t, act, div, pb, pdet, pdt,
-                                        [&](int r) { return VIS || !(pnb[r] < 0 || (inBlock(pnb[r]) && !a.fullTraces)); });
+  // (4) correction of the jump (correctDivFlux, solver.cpp:789-806) and the
+  // stage update; the updated state goes to sFd (free after (2)) for its
+  // traces, so that sU keeps the stage state other elements of the block read.
+  // (4) and (5) stand here and once more in the viscous update (viscUpdate):
+  // called as one function, they came out with other code that took FP32 hex P3
+  // with the metrics formed in the kernel from 66 to 69 us a stage at 32^3 and
+  // from 224 to 234 at 48^3, whatever its arguments and register count.
+  T utv[NF];  // the updated state at this thread's point, for the traces of (5)
+  if (hasS) {
+    int cq[NFACE], cside[NFACE], cax[NFACE];
+    corrEntries<D, P>(t, cq, cside, cax);
+    T cw[NFACE];  // correction weights, read once for all fields
+#pragma unroll
+    for (int f = 0; f < NFACE; f++) cw[f] = s1[(cside[f] ? O::GR : O::GL) + cax[f]];
+    const size_t eo = (size_t)e * NF * NS;
+#pragma unroll
+    for (int k = 0; k < NF; k++) {
+      T corr = (T)0;
+#pragma unroll
+      for (int f = 0; f < NFACE; f++) corr += cw[f] * sJ[slot][k][cq[f]];
+      const T dv = corr + div[k];
+      const size_t gi = eo + (size_t)k * NS + t;
+      if (a.divF) __builtin_nontemporal_store(dv, a.divF + gi);
+      if (!FIN && a.mode == 0) continue;
+      // stage terms RK * divF / detJ * dt, with dt / detJ formed once per point
+      const double dtJ = pdt / pdet;
+      double u = pb[k];
+      // DEF: the base state read again here instead of kept in registers
+      if constexpr (DEF) u = (double)a.UbaseT[gi];
+      if (FIN && a.mode == 2) {
+        // earlier residuals: already subtracted from pb (before the barrier)
+        const double cl = (a.nprev == 0) ? a.c0 : (a.nprev == 1) ? a.c1 : (a.nprev == 2) ? a.c2 : a.c3;
+        u -= cl * (double)dv * dtJ;
+      } else {
+        u = u - a.rk * (double)dv * dtJ;
+      }
+      // the updated state in the residual precision, for the traces: FP32
+      // states hold the energy less Phys::eOff, and the final stages' FP64
+      // base (hence u) is absolute
+      double ut = u;
+      if constexpr (hasEnergyOffset<T>())
+        if (k == NF - 1 && base64) ut = u - a.ph.eOff;
+      if constexpr (!FIN) {
+        if (a.Unext) __builtin_nontemporal_store((T)u, a.Unext + gi);
+      } else {
+        __builtin_nontemporal_store(u, a.Uout + gi);
+        if (a.Uout32) __builtin_nontemporal_store((float)ut, a.Uout32 + gi);
+      }
+      sFd[slot][k][tP] = (T)ut;
+      utv[k] = (T)ut;
+    }
+  }
+  if (!FIN && a.mode == 0) return;
+  elementSync<TPE>();
+
+  // (5) face traces of the updated state for the next stage, for the faces
+  // whose neighbour is in another block
+  if (act) {
+    T *Fe = a.UfOut + (size_t)e * NF * NFP;
+#pragma unroll
+    for (int r = 0; r < NQ; r++) {
+      const int q = fq(r);
+      T tv[NF];
+      if constexpr (MFF) mfmaFaceRound<NF, G::NSP, T>(s1, &sFd[slot][0][0], t, utv, r, tv);
+      if (q >= NFP) continue;
+      if (!VIS && (pnb[r] < 0 || (inBlock(pnb[r]) && !a.fullTraces))) continue;
+      if constexpr (MFF) {
+#pragma unroll
+        for (int k = 0; k < NF; k++) __builtin_nontemporal_store(tv[k], Fe + k * NFP + q);
+        continue;
+      }
+      int base, stride, side, dn;
+      fptLine<D, P>(q, base, stride, side, dn);
+      const int lb = padIdx<P>(base), ls = padStride<P>(stride);
+      const T *l1 = s1 + (side ? O::LR : O::LL);
+#pragma unroll
+      for (int k = 0; k < NF; k++) {
+        T acc = (T)0;
+#pragma unroll
+        for (int m = 0; m < P1; m++) acc += l1[m] * sFd[slot][k][lb + m * ls];
+        __builtin_nontemporal_store(acc, Fe + k * NFP + q);
+      }
+    }
+  }
 }
 
 // The inviscid final-stage variant asks for 3 waves per SIMD (at most 168

@@ -302,8 +302,95 @@ __global__ __launch_bounds__((ElemGeo<D, P>::NTH), 2) void k_visc_flux(StageArgs
     for (int k = 0; k < NF; k++) a.divW[((size_t)e * NF + k) * NS + t] = div[k];
 }
 
+// The end of a viscous stage, as phases (4) and (5) of stageBody: the correction of the
+// jumps sJe [NF][NFP] (correctDivFlux, solver.cpp:789-806) added to the
+// divergence div, the stage update from the base pb (final stages: with the
+// earlier residuals' terms already subtracted), and the face traces of the
+// updated state, staged in sSe [NF][NSP].
+template <int D, int P, int NF, typename T, bool FIN>
+__device__ __forceinline__ void viscUpdate(const StageArgs<T> &a, const T *s1, const T *sJe, T *sSe, const int e,
+                                           const int t, const bool act, const T *div, const double *pb,
+                                           const double pdet, const double pdt) {
+  using G = ElemGeo<D, P>;
+  using O = OneD<P>;
+  constexpr int NS = G::NS, NSP = G::NSP, NFP = G::NFP, P1 = G::P1, TPE = G::TPE, NFACE = G::NFACE;
+  constexpr int NQ = (NFP + TPE - 1) / TPE;
+  constexpr bool MF = FR_MFMA && D == 3 && P == 3, MFF = MF && sizeof(T) == 8;
+  // the FP64 base of the final stages is absolute; FP32 stage states hold the
+  // energy less Phys::eOff
+  constexpr bool base64 = FIN;
+  T utv[NF];  // the updated state at this thread's point
+  if (act && t < NS) {
+    int cq[NFACE], cside[NFACE], cax[NFACE];
+    corrEntries<D, P>(t, cq, cside, cax);
+    T cw[NFACE];  // correction weights, read once for all fields
+#pragma unroll
+    for (int f = 0; f < NFACE; f++) cw[f] = s1[(cside[f] ? O::GR : O::GL) + cax[f]];
+    const size_t eo = (size_t)e * NF * NS;
+#pragma unroll
+    for (int k = 0; k < NF; k++) {
+      T corr = (T)0;
+#pragma unroll
+      for (int f = 0; f < NFACE; f++) corr += cw[f] * sJe[k * NFP + cq[f]];
+      const T dv = corr + div[k];
+      const size_t gi = eo + (size_t)k * NS + t;
+      if (a.divF) __builtin_nontemporal_store(dv, a.divF + gi);
+      if (!FIN && a.mode == 0) continue;
+      // stage terms RK * divF / detJ * dt, with dt / detJ formed once per point
+      const double dtJ = pdt / pdet;
+      double u = pb[k];
+      if (FIN && a.mode == 2) {
+        // earlier residuals: already subtracted from pb
+        const double cl = (a.nprev == 0) ? a.c0 : (a.nprev == 1) ? a.c1 : (a.nprev == 2) ? a.c2 : a.c3;
+        u -= cl * (double)dv * dtJ;
+      } else {
+        u = u - a.rk * (double)dv * dtJ;
+      }
+      // the updated state in the residual precision, for the traces
+      double ut = u;
+      if constexpr (hasEnergyOffset<T>())
+        if (k == NF - 1 && base64) ut = u - a.ph.eOff;
+      if constexpr (!FIN) {
+        if (a.Unext) __builtin_nontemporal_store((T)u, a.Unext + gi);
+      } else {
+        __builtin_nontemporal_store(u, a.Uout + gi);
+        if (a.Uout32) __builtin_nontemporal_store((float)ut, a.Uout32 + gi);
+      }
+      sSe[k * NSP + padIdx<P>(t)] = (T)ut;
+      utv[k] = (T)ut;
+    }
+  }
+  if (!FIN && a.mode == 0) return;
+  elementSync<TPE>();
+  if (!act) return;
+  T *Fe = a.UfOut + (size_t)e * NF * NFP;
+#pragma unroll
+  for (int r = 0; r < NQ; r++) {
+    const int q = MF ? mfmaFpt(t, r) : t + r * TPE;
+    T tv[NF];
+    if constexpr (MFF) mfmaFaceRound<NF, NSP, T>(s1, sSe, t, utv, r, tv);
+    if (q >= NFP) continue;
+    if constexpr (MFF) {
+#pragma unroll
+      for (int k = 0; k < NF; k++) __builtin_nontemporal_store(tv[k], Fe + k * NFP + q);
+      continue;
+    }
+    int base, stride, side, dn;
+    fptLine<D, P>(q, base, stride, side, dn);
+    const int lb = padIdx<P>(base), ls = padStride<P>(stride);
+    const T *l1 = s1 + (side ? O::LR : O::LL);
+#pragma unroll
+    for (int k = 0; k < NF; k++) {
+      T acc = (T)0;
+#pragma unroll
+      for (int m = 0; m < P1; m++) acc += l1[m] * sSe[k * NSP + lb + m * ls];
+      __builtin_nontemporal_store(acc, Fe + k * NFP + q);
+    }
+  }
+}
+
 // The second half of a viscous stage: the common flux from the two sides'
-// shares, then the end of the stage as in the inviscid kernel (stageUpdate).
+// shares, then the end of the stage as in the inviscid kernel (viscUpdate).
 // Bound by its bytes (the shares, the divergence, the base and the outputs);
 // no element reads another's LDS, so beyond the barrier for the 1D table the
 // elements of a workgroup run on their own.
@@ -376,8 +463,7 @@ __global__ __launch_bounds__((ElemGeo<D, P>::NTH)) void k_visc_update(StageArgs<
   if constexpr (FIN)
     if (a.mode == 2) subtractEarlier<NF, T>(a, pd, pdt / pdet, pb);
   __syncthreads();
-  stageUpdate<D, P, NF, T, FIN, false, 0>(a, s1, &sJ[slot][0][0], &sS[slot][0][0], e, t, act, div, pb, pdet, pdt,
-                                          [](int) { return true; });
+  viscUpdate<D, P, NF, T, FIN>(a, s1, &sJ[slot][0][0], &sS[slot][0][0], e, t, act, div, pb, pdet, pdt);
 }
 
 }  // namespace frdev
