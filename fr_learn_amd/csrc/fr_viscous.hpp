@@ -24,9 +24,10 @@
 // point) moved 11.5 KB out, 23 KB in and, with the common flux formed by a
 // launch of its own, 77 KB per element and stage in all against 35 KB.
 // Navier-Stokes 24^3 P3 (13824 elements, FP64): a stage took 61 us (gradient)
-// + 61 (common flux) + 88 (stage) and takes 70 (k_visc_flux, bound by its
-// vector instructions at two waves per SIMD; three spill 20 registers and ran
-// 83 us) + 41 (k_visc_update, 57 in the final stage; bound by its bytes).
+// + 61 (common flux) + 88 (stage) and takes 60 (k_visc_flux: LDS and latency at
+// two waves per SIMD; three spill 20 registers and ran 83 us) + 41
+// (k_visc_update, 57 in the final stage; bound by its bytes, 6.9 TB/s with the
+// caches).
 #pragma once
 
 #include "fr_kernels.hpp"
@@ -120,10 +121,16 @@ __global__ __launch_bounds__((ElemGeo<D, P>::NTH), 2) void k_visc_flux(StageArgs
   // (0) at every flux point the LDG jump, and what both sides form alike of
   // the common flux
   T I[SH ? NQ : 1][NF];
+  // matrix cores: the state at the lane's flux points, kept for (2) (20 registers
+  // below the limit of two waves; formed again there, a stage of Navier-Stokes
+  // 24^3 P3 took 116.5 us on average against 114.0, 40^3 547 against 537.
+  // Staging the gradient in LDS for (2) as well, instead of lane pulls, gained
+  // nothing: 114.5 and 540)
+  T uf[MG ? NQ : 1][NF];
 #pragma unroll
   for (int r = 0; r < NQ; r++) {
     const int q = fq(r);
-    T uo[NF];
+    T(&uo)[NF] = uf[MG ? r : 0];
     if (MG && act) ownTrace(r, q, uo);
     if (act && q < NFP) {
       if (!MG) ownTrace(r, q, uo);
@@ -190,12 +197,12 @@ __global__ __launch_bounds__((ElemGeo<D, P>::NTH), 2) void k_visc_flux(StageArgs
 #pragma unroll
   for (int r = 0; r < NQ; r++) {
     const int q = fq(r);
-    T gf[D][NF], uo[NF];
+    T gf[D][NF];
+    T(&uo)[NF] = uf[MG ? r : 0];
     if constexpr (MG) {
       if (act) {
 #pragma unroll
         for (int d = 0; d < D; d++) mfmaFaceRoundReg<NF, T>(s1, t, g[d], r, gf[d]);
-        if (SH) ownTrace(r, q, uo);
       }
     }
     if (!act || q >= NFP) continue;
