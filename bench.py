@@ -309,7 +309,7 @@ def tgv_ns_adjoint(n=24, steps=200, every=20, eps=1e-6, seed=0):
                 "gradient_and_face_flux_ms": gr_ms / max(gr_n, 1), "stage_kernel_ms": st_ms / max(st_n, 1),
                 "achieved": b_vis / (stage_ms * 1e-3) / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                 "frac": b_vis / (stage_ms * 1e-3) / HBM_PEAK,
-                "note": "k_grad + k_vflux + k_stage<...,VIS> per RK stage (HIP events); bytes = B_res + "
+                "note": "k_visc_flux + k_visc_update per RK stage (HIP events); bytes = B_res + "
                         "E*Ns*2*D*Nf*s"},
             "fd_directional": fd, "adjoint_directional": adj, "rel_diff_vs_fd": abs(fd - adj) / abs(fd),
             "eps": eps}
