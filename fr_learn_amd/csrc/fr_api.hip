@@ -260,7 +260,7 @@ RefChunk refChunk(const fr_ctx *c, int NF, int NP, int most) {
   r.lds = r.et * row;
   return r;
 }
-// Points of all elements' NF fields that Us holds.
+// Points of all elements' NF fields that Us holds (one at least, by its size).
 int usPoints(const fr_ctx *c, int NF) {
   return (int)std::max<size_t>(1, c->nState() * c->tsize() / 8 / ((size_t)c->nE * NF));
 }
@@ -678,12 +678,15 @@ int createImpl(const fr_config *cfg, const fr_mesh *m, int precision, fr_ctx *c)
   HIP_TRY(hipMemset(c->U0, 0, nSt * 8));
   const size_t ts = c->tsize();
   for (int b = 0; b < 2; b++) HIP_TRY(hipMalloc(&c->Uf[b], (size_t)nE * c->NF * NFP * ts));
-  HIP_TRY(hipMalloc(&c->Us, nSt * ts));
+  // at least one point of any array that changes layout through it (usPoints):
+  // NF or, the normals, D fields of 8 bytes an element
+  const size_t usBytes = std::max(nSt * ts, (size_t)nE * std::max(c->NF, D) * 8);
+  HIP_TRY(hipMalloc(&c->Us, usBytes));
   if ((rc = dmalloc(&c->dtG, 1))) return rc;
   HIP_TRY(hipMemcpy(c->dtG, &cfg->dt, sizeof(double), hipMemcpyHostToDevice));
   if (cfg->viscous)
     HIP_TRY(hipMalloc(&c->Gv, (size_t)nE * c->NF * NFP * ts));
-  HIP_TRY(hipMemset(c->Us, 0, nSt * ts));
+  HIP_TRY(hipMemset(c->Us, 0, usBytes));
   for (int s = 0; s < c->nRK; s++) {
     HIP_TRY(hipMalloc(&c->divF[s], nSt * ts));
     HIP_TRY(hipMemset(c->divF[s], 0, nSt * ts));

@@ -48,6 +48,21 @@ def test_state_layouts(elem, P, n, equation, precision):
     g.close()
 
 
+def test_scratch_holds_a_point_of_the_normals():
+    """The smallest stage state, 3 FP32 values an element, against the 2 FP64
+    components of a normal, on a mesh whose normals pass the pinned buffer's
+    size: the same array as from an FP64 context, bit for bit."""
+    n = (310, 290)
+    m = mesh.tri_box(n, (0.0, 0.0), (1.0, 1.0), perturb=0.2, seed=1)
+    out = []
+    for precision in ("fp32", "fp64"):
+        g = Solver(cases.config(nDims=2, order=1, equation=0), m, precision=precision)
+        out.append(g.geometry(2))
+        g.close()
+    assert out[0].nbytes > 8 << 20
+    assert np.array_equal(out[0], out[1])
+
+
 def test_read_backs_from_several_threads():
     """The pinned buffer is one for the process: threads that meet at it get
     their own context's state."""
