@@ -635,7 +635,7 @@ struct StageSmem {
   // Hex P3 keeps them in registers (matrix cores).  These meshes wait on the
   // chain of LDS phases, not on bytes: with one synchronisation for two an axis,
   // P5 hexes (17 x 15 x 13, FP64, 200 steps of RK4) took 37.7 -> 35.4 ms, 40 mixed
-  // small meshes in one graph 28.4 -> 26.9, P4 quads (128^2) 38.9 -> 38.5.
+  // small meshes in one graph 28.4 -> 26.9; P4 quads (128^2) did not change.
   static constexpr bool MF = FR_MFMA && D == 3 && P == 3;
   static constexpr bool SHARE = !MF && D == 3 && G::NFP >= G::NSP;
   static constexpr int NX = MF ? 0 : D - 1 - (SHARE ? 1 : 0);
