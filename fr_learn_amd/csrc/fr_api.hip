@@ -1124,6 +1124,9 @@ int fr_get_array(fr_ctx *c, int which, double *out) {
   }
   // the residual's face fluxes store new wave speeds, as in residual()
   if (c->dtType != 0 && !c->dtFirst && !c->dtFrozen) c->dtReady = false;
+  // the debug kernel's element blocks are those of tile layout 0, the last
+  // update's need not be (stageTile): extrapolate afresh, every face
+  c->traceOf = -1;
   int rc = ensureTraces<double>(c, 0);
   if (!rc) {
     frdev::StageArgs<double> a = makeStageArgs<double>(c, 0, c->cur, 0, 0, 0.0);
