@@ -800,6 +800,14 @@ int createImpl(const fr_config *cfg, const fr_mesh *m, int precision, fr_ctx *c)
       hipLaunchKernelGGL(frdev::k_affine<2>, dim3(nblk(nE)), dim3(256), 0, c->stream, c->JG64, c->detJ, c->fgeo64,
                          NS, NFP, c->NFPF, c->NFACE, nE, tol, c->JGc64, c->detJc, c->fgeoc64, dOk);
     HIP_TRY(hipGetLastError());
+    const long nf = (long)nE * c->NFACE;
+    if (D == 3)
+      hipLaunchKernelGGL(frdev::k_affine_right<3>, dim3(nblk(nf)), dim3(256), 0, c->stream, c->fnbr, c->finfo,
+                         c->NFACE, nE, c->fgeoc64);
+    else
+      hipLaunchKernelGGL(frdev::k_affine_right<2>, dim3(nblk(nf)), dim3(256), 0, c->stream, c->fnbr, c->finfo,
+                         c->NFACE, nE, c->fgeoc64);
+    HIP_TRY(hipGetLastError());
     std::vector<int8_t> ok(nE);
     HIP_TRY(hipMemcpyAsync(ok.data(), dOk, nE, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));

@@ -1608,6 +1608,23 @@ __global__ void k_affine(const double *__restrict__ JG, const double *__restrict
   ok[e] = good ? 1 : 0;
 }
 
+// The compact normal of a face's right element is its left element's entry,
+// bit for bit (k_affine took the left normal at another point of the face
+// there, equal but for rounding): the two sides' shares of the viscous common
+// flux add up to it only if both take the same side of the LDG switch
+// (ldgPenalty), also where n.(1, 1, sqrt 2) is zero but for rounding.  One
+// thread per (element, face); left entries are not written.
+template <int D>
+__global__ void k_affine_right(const int32_t *__restrict__ fnbr, const int8_t *__restrict__ finfo, int nFace,
+                               int nEles, double *fgeoc) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (long)nEles * nFace) return;
+  const int fi = finfo[i];
+  if (fi >= FINFO_BOUNDARY || !((fi >> 5) & 1)) return;
+  const long e = i / nFace, f = i - e * nFace, l = fnbr[i];
+  for (int c = 0; c < D; c++) fgeoc[(e * (D + 1) + c) * nFace + f] = fgeoc[(l * (D + 1) + c) * nFace + (fi & 7)];
+}
+
 static __global__ void k_to_float(const double *__restrict__ a, float *__restrict__ b, long n) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) b[i] = (float)a[i];
