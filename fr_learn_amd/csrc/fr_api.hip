@@ -327,14 +327,14 @@ int refToDev(fr_ctx *c, const double *src, double *dst, int NF, int NP) {
   HIP_TRY(hipStreamSynchronize(c->stream));
   return 0;
 }
-template <typename TD>
+template <bool ADD = false, typename TD>
 int devToRef(fr_ctx *c, const TD *src, double *dst, int NF, int NP, double add = 0.0) {
   const RefChunk r = refChunk(c, NF, NP, usPoints(c, NF));
   const size_t plane = (size_t)c->nE * NF;
   std::unique_lock<std::mutex> lock(gStage.m, std::defer_lock);
   if (double *buf = stageBuffer(lock, plane * NP * 8)) {
     const RefChunk w = refChunk(c, NF, NP, NP);
-    hipLaunchKernelGGL(frdev::k_to_ref<TD>, dim3((c->nE + w.et - 1) / w.et), dim3(256), w.lds, c->stream, src,
+    hipLaunchKernelGGL((frdev::k_to_ref<TD, ADD>), dim3((c->nE + w.et - 1) / w.et), dim3(256), w.lds, c->stream, src,
                        c->ipermD, NF, NP, c->nE, w.et, 0, NP, add, buf);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(c->stream));
@@ -343,7 +343,7 @@ int devToRef(fr_ctx *c, const TD *src, double *dst, int NF, int NP, double add =
   }
   for (int p = 0; p < NP; p += r.pts) {
     const int np = std::min(r.pts, NP - p);
-    hipLaunchKernelGGL(frdev::k_to_ref<TD>, dim3((c->nE + r.et - 1) / r.et), dim3(256), r.lds, c->stream, src,
+    hipLaunchKernelGGL((frdev::k_to_ref<TD, ADD>), dim3((c->nE + r.et - 1) / r.et), dim3(256), r.lds, c->stream, src,
                        c->ipermD, NF, NP, c->nE, r.et, p, np, add, (double *)c->Us);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpyAsync(dst + p * plane, c->Us, np * plane * 8, hipMemcpyDeviceToHost, c->stream));
@@ -1175,7 +1175,7 @@ int fr_get_traces(fr_ctx *c, double *out) {
   int rc = (c->prec == FR_PREC_FP32) ? ensureTraces<float>(c, 0) : ensureTraces<double>(c, 0);
   if (rc) return rc;
   // the FP32 energy traces are offset (Phys::eOff)
-  return c->prec == FR_PREC_FP32 ? devToRef(c, (const float *)c->Uf[c->cur], out, c->NF, c->NFP, c->ph.eOff)
+  return c->prec == FR_PREC_FP32 ? devToRef<true>(c, (const float *)c->Uf[c->cur], out, c->NF, c->NFP, c->ph.eOff)
                                  : devToRef(c, (const double *)c->Uf[c->cur], out, c->NF, c->NFP);
 }
 

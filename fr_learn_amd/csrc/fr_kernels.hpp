@@ -1412,8 +1412,9 @@ static __global__ void k_state_to_float(const double *__restrict__ U, float *__r
 // point.  The copy to the host bounds a read-back (17 GB/s into pageable
 // memory): the 283 MB state of 48^3 P3 takes 27 ms with a fresh host array and
 // took 263 ms with the layout changed by a host loop, whose every access missed
-// the cache.  add (FP32 energies, Phys::eOff) goes to the last field.
-template <typename TD>
+// the cache.  Copies keep every bit; with ADD (FP32 traces) add is added to the
+// last field (Phys::eOff).
+template <typename TD, bool ADD>
 __global__ __launch_bounds__(256) void k_to_ref(const TD *__restrict__ src, const int *__restrict__ iperm, int NF,
                                                 int NP, int nE, int ET, int p0, int np, double add,
                                                 double *__restrict__ ref) {
@@ -1421,7 +1422,9 @@ __global__ __launch_bounds__(256) void k_to_ref(const TD *__restrict__ src, cons
   const int e0 = blockIdx.x * ET, ne = min(ET, nE - e0), st = np | 1;
   for (int i = threadIdx.x; i < ne * NF * np; i += blockDim.x) {
     const int r = i / np, p = i - r * np, e = r / NF, k = r - e * NF;
-    tile[r * st + p] = (double)src[((size_t)iperm[e0 + e] * NF + k) * NP + p0 + p] + (k == NF - 1 ? add : 0.0);
+    double v = (double)src[((size_t)iperm[e0 + e] * NF + k) * NP + p0 + p];
+    if constexpr (ADD) v += k == NF - 1 ? add : 0.0;
+    tile[r * st + p] = v;
   }
   __syncthreads();
   const int run = ne * NF;

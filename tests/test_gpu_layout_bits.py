@@ -17,7 +17,7 @@ ODD = np.array([0x8000000000000000, 0x0000000000000001, 0x800fffffffffffff, 0x7f
 def test_state_bits(D, P, n, equation):
     g = Solver(cases.config(nDims=D, order=P, equation=equation), mesh.box(D, n, (0.0,) * D, (1.0,) * D))
     U = np.random.default_rng(1).uniform(1.0, 2.0, g.state_shape())
-    # all but the last field's first entries odd: the energy as well as the first field
+    # odd entries in every field
     flat = U.reshape(-1, g.nFields)
     for k in range(g.nFields):
         flat[k:k + 3 * len(ODD):3, k] = ODD
