@@ -541,7 +541,7 @@ int stageStates(fr_ctx *c, const double **S) {
     a.rprev = nullptr;
     a.UfIn = c->adjTr[s];
     a.UfOut = c->adjTr[s + 1];
-    a.fullTraces = 1;
+    a.mode = frdev::MODE_TRACES;
     a.divF = nullptr;
     a.divW = c->adjNu;  // written by vjpStepDev after this
     a.Unext = c->adjS[s + 1];
