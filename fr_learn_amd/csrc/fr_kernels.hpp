@@ -532,25 +532,6 @@ __device__ __forceinline__ void mfmaFaceRoundReg(const T *s1, const int t, const
                   : V::ext(L.aEzy, lanePull(L.by, own[k]), (T)0);
 }
 
-// The physical gradient JGinv^T gr / detJ of a reference-space gradient gr at
-// one point, J = JGinv(dimRef, dimPhys).
-template <int D, int NF, typename T>
-__device__ __forceinline__ void physicalGradient(const T gr[D][NF], const T *J, T detJ, T g[D][NF]) {
-  const T invDet = recip(detJ);
-#pragma unroll
-  for (int d1 = 0; d1 < D; d1++) {
-    T Jd[D];
-#pragma unroll
-    for (int d = 0; d < D; d++) Jd[d] = J[d * D + d1] * invDet;
-#pragma unroll
-    for (int k = 0; k < NF; k++) {
-      T acc = gr[0][k] * Jd[0] + gr[1][k] * Jd[1];
-      if constexpr (D == 3) acc = acc + gr[2][k] * Jd[2];
-      g[d1][k] = acc;
-    }
-  }
-}
-
 // correctedGradient (below) for hex P3 with the reference-space derivative on
 // the matrix cores: the state S in LDS (fields RS apart, padded rows when
 // PADV) and the lane's own values own[], the jumps sCe [NF][NFP] at flux

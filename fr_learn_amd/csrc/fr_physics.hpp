@@ -433,12 +433,20 @@ __device__ __forceinline__ void viscousFlux(const Phys &ph, const T *U, const TG
     //   grad e = (grad E - (E / rho) grad rho) / rho - sum_c v_c grad v_c,
     // which is the reference's grad E - grad(rho |v|^2 / 2) - e grad rho
     // regrouped; the ratio gamma / Pr and the third of the divergence are
-    // constants.  Ulp-level differences.
-    const T ri = recip(U[0]);
+    // constants.  Ulp-level differences.  FP32 divides by rho and by 3: with
+    // the products the rounding error of its momentum flux was 7-15 % larger
+    // (random states of order one with density gradients), with the divisions
+    // it is below that of the reference's grouping.
+    constexpr bool F64 = sizeof(T) == 8;
+    const T ri = F64 ? recip(U[0]) : (T)0;
+    auto over = [&](const T &x) -> T {
+      if constexpr (F64) return x * ri;
+      else return x / U[0];
+    };
     T v[D];
 #pragma unroll
-    for (int c = 0; c < D; c++) v[c] = U[c + 1] * ri;
-    const T H = U[D + 1] * ri;
+    for (int c = 0; c < D; c++) v[c] = over(U[c + 1]);
+    const T H = over(U[D + 1]);
     T mu = (T)ph.mu_inf;
     if (!ph.fixVis) {  // Sutherland's law
       T q = v[0] * v[0];
@@ -447,7 +455,7 @@ __device__ __forceinline__ void viscousFlux(const Phys &ph, const T *U, const TG
       const T rt = ((T)ph.gamma - (T)1.0) * (H - (T)0.5 * q) / (T)ph.rt_inf;
       mu *= pow(rt, (T)1.5) * ((T)1. + (T)ph.c_sth) / (rt + (T)ph.c_sth);
     }
-    const T mr = mu * ri;  // mu / rho: the stresses need mu grad v
+    const T mr = over(mu);  // mu / rho: the stresses need mu grad v
     // G[d][c] = mu dv_c/dx_d and h[d] = mu de/dx_d
     T G[D][D], h[D];
 #pragma unroll
@@ -460,7 +468,7 @@ __device__ __forceinline__ void viscousFlux(const Phys &ph, const T *U, const TG
     }
     T diag = G[0][0] + G[1][1];
     if constexpr (D == 3) diag += G[2][2];
-    diag = diag * (T)(1.0 / 3.0);
+    diag = F64 ? diag * (T)(1.0 / 3.0) : diag / (T)3.0;
     const T kq = (T)(ph.gamma / ph.prandtl);
     T tau[D][D];  // tau[d][c], symmetric
 #pragma unroll
@@ -482,6 +490,27 @@ __device__ __forceinline__ void viscousFlux(const Phys &ph, const T *U, const TG
     }
     if constexpr (D == 3)
       if (!ph.viscFix) Fv[0][3] = -tau[2][2];
+  }
+}
+
+// The physical gradient JGinv^T gr / detJ of a reference-space gradient gr at
+// one point, J = JGinv(dimRef, dimPhys).  FP64: one reciprocal (recip) folded
+// into the metrics; FP32 divides, after the sum.
+template <int D, int NF, typename T>
+__device__ __forceinline__ void physicalGradient(const T gr[D][NF], const T *J, T detJ, T g[D][NF]) {
+  constexpr bool F64 = sizeof(T) == 8;
+  const T invDet = F64 ? recip(detJ) : (T)1 / detJ;
+#pragma unroll
+  for (int d1 = 0; d1 < D; d1++) {
+    T Jd[D];
+#pragma unroll
+    for (int d = 0; d < D; d++) Jd[d] = F64 ? J[d * D + d1] * invDet : J[d * D + d1];
+#pragma unroll
+    for (int k = 0; k < NF; k++) {
+      T acc = gr[0][k] * Jd[0] + gr[1][k] * Jd[1];
+      if constexpr (D == 3) acc = acc + gr[2][k] * Jd[2];
+      g[d1][k] = F64 ? acc : invDet * acc;
+    }
   }
 }
 
