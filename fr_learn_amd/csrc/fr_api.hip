@@ -33,8 +33,7 @@ void freeAll(fr_ctx *c) {
                   c->adjLam,  c->adjOut,  c->adjNu,   c->adjW,    c->adjS[0], c->adjS[1],
                   c->adjS[2], c->adjS[3], c->adjB,    c->JGc64,  c->detJc, c->fgeoc64,
                   c->JGc32,   c->fgeoc32, c->waveSp,
-                  c->dtNum,   c->wsurf,   c->dtPart,  c->geoN64,  c->geoN32,  c->errTab, c->Xd,
-                  c->ipermD};
+                  c->dtNum,   c->wsurf,   c->dtPart,  c->geoN64,  c->geoN32,  c->errTab, c->Xd};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   for (auto &v : c->ev)
@@ -266,10 +265,11 @@ int usPoints(const fr_ctx *c, int NF) {
 }
 
 // Small arrays go through pinned host memory that the layout kernels access
-// themselves: one buffer for the process, made by the first of them and
-// freed with the last context.  A copy into the caller's pageable array costs the runtime
-// its pinning, most of all where the array is fresh, and a wait of its own
-// behind a busy stream: 74 KB 35 -> 6.5 us, 524 KB 60 -> 27 us, 40 arrays of
+// themselves: one buffer for the process, made and grown by the arrays that
+// pass it (a small solver's first one waits 10 us less than for 8 MB at once),
+// freed with the last context.  A copy into the caller's pageable array costs
+// the runtime its pinning, most of all where the array is fresh, and a wait of
+// its own behind a busy stream: 74 KB 35 -> 6.5 us, 524 KB 60 -> 27 us, 40 arrays of
 // 0.65 MB 15 -> 9 ms fresh and 8.4 -> 4.3 ms reused.  From some MB on both move
 // 17 GB/s, so larger arrays are copied and the buffer stays small.  A thread that
 // finds the buffer in use takes the copy.
@@ -277,29 +277,38 @@ constexpr size_t kStageBytes = 8u << 20;
 struct HostStage {
   std::mutex m;
   double *buf = nullptr;
+  size_t size = 0;
   int contexts = 0;
 };
 HostStage gStage;
+void stageFree() {
+  if (gStage.buf) (void)hipHostFree(gStage.buf);
+  gStage.buf = nullptr;
+  gStage.size = 0;
+}
 void stageRetain() {
   std::lock_guard<std::mutex> lock(gStage.m);
   gStage.contexts++;
 }
 void stageRelease() {
   std::lock_guard<std::mutex> lock(gStage.m);
-  if (--gStage.contexts == 0 && gStage.buf) {
-    (void)hipHostFree(gStage.buf);
-    gStage.buf = nullptr;
-  }
+  if (--gStage.contexts == 0) stageFree();
 }
 
 // The buffer, held until the lock goes, or null: bytes too large, in use, or not
 // to be had.
 double *stageBuffer(std::unique_lock<std::mutex> &lock, size_t bytes) {
   if (bytes > kStageBytes || !lock.try_lock()) return nullptr;
-  if (!gStage.buf &&
-      hipHostMalloc((void **)&gStage.buf, kStageBytes, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
-    gStage.buf = nullptr;
-    (void)hipGetLastError();
+  if (gStage.size < bytes) {
+    stageFree();
+    size_t size = 64u << 10;
+    while (size < bytes) size *= 2;
+    if (hipHostMalloc((void **)&gStage.buf, size, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess) {
+      gStage.size = size;
+    } else {
+      gStage.buf = nullptr;
+      (void)hipGetLastError();
+    }
   }
   return gStage.buf;
 }
@@ -671,7 +680,7 @@ int createImpl(const fr_config *cfg, const fr_mesh *m, int precision, fr_ctx *c)
   if ((rc = dmalloc(&c->U, nSt)) || (rc = dmalloc(&c->U0, nSt)) || (rc = dmalloc(&c->detJ, (size_t)nE * NS)) ||
       (rc = dmalloc(&c->JG64, (size_t)nE * D * D * NS)) || (rc = dmalloc(&c->fgeo64, (size_t)nE * (D + 1) * NFP)) ||
       (rc = dmalloc(&c->ownN, (size_t)nE * D * NFP)) || (rc = dmalloc(&c->wts, NS)) ||
-      (rc = dmalloc(&c->oned64, c->ops.oned.size())) || (rc = dmalloc(&c->fnbr, (size_t)nE * c->NFACE)) ||
+      (rc = dmalloc(&c->oned64, c->ops.oned.size())) || (rc = dmalloc(&c->fnbr, (size_t)nE * (c->NFACE + 1))) ||
       (rc = dmalloc(&c->finfo, (size_t)nE * c->NFACE)))
     return rc;
   HIP_TRY(hipMemset(c->U, 0, nSt * 8));
@@ -715,8 +724,6 @@ int createImpl(const fr_config *cfg, const fr_mesh *m, int precision, fr_ctx *c)
     for (int i = 0; i < nE; i++) c->iperm[c->perm[i]] = i;
     for (int e = 0; e < nE; e++)
       if (c->iperm[e] < 0) return fail(FR_EMESH, "element order is not a permutation");
-    if ((rc = dmalloc(&c->ipermD, (size_t)nE))) return rc;
-    HIP_TRY(hipMemcpy(c->ipermD, c->iperm.data(), (size_t)nE * sizeof(int), hipMemcpyHostToDevice));
   }
   // geometry on device
   {
@@ -743,7 +750,7 @@ int createImpl(const fr_config *cfg, const fr_mesh *m, int precision, fr_ctx *c)
     {
       // per-element tables in device order, neighbour ids renumbered
       const int NFACE = c->NFACE;
-      std::vector<int32_t> pe((size_t)nE * NFP), fn((size_t)nE * NFACE);
+      std::vector<int32_t> pe((size_t)nE * NFP), fn((size_t)nE * (NFACE + 1));
       std::vector<int8_t> fi((size_t)nE * NFACE);
       for (int de = 0; de < nE; de++) {
         const size_t e = (size_t)c->perm[de];
@@ -757,6 +764,11 @@ int createImpl(const fr_config *cfg, const fr_mesh *m, int precision, fr_ctx *c)
           fi[(size_t)de * NFACE + f] = c->conn.finfo[e * NFACE + f];
         }
       }
+      // the element order rides behind the neighbours: with an allocation and an
+      // upload of its own, a solver of 64 quads was created in 0.51 ms instead
+      // of 0.42 (medians of six)
+      std::copy(c->iperm.begin(), c->iperm.end(), fn.begin() + (size_t)nE * NFACE);
+      c->ipermD = c->fnbr + (size_t)nE * NFACE;
       HIP_TRY(hipMemcpy(pairEF, pe.data(), pe.size() * 4, hipMemcpyHostToDevice));
       HIP_TRY(hipMemcpy(c->finfo, fi.data(), fi.size(), hipMemcpyHostToDevice));
       HIP_TRY(hipMemcpy(c->fnbr, fn.data(), fn.size() * 4, hipMemcpyHostToDevice));

@@ -124,7 +124,7 @@ struct fr_ctx {
   std::vector<double> X;  // host copy of element node coordinates [device ele][node][3]
   std::vector<int> perm;  // device element -> mesh element (blocks of EPB face-connected elements)
   std::vector<int> iperm; // mesh element -> device element
-  int *ipermD = nullptr;  // the same on the device
+  int *ipermD = nullptr;  // the same on the device (behind fnbr, not freed by itself)
   int epb = 1;
   bool tri = false;  // linear triangles (fr_tri_ops.cpp / fr_tri.hpp)
   // timing
