@@ -478,9 +478,9 @@ __global__ __launch_bounds__((VjpTile<D, P>::NTH), (P == 3 && !BND) ? 2 : 1) voi
   const int sk = D == 3 ? tc / (P1 * P1) : 0, sj = (tc / P1) % P1, si = tc % P1;
   if (MG ? act : hasS) {
     if constexpr (MG) {
-      mfmaGradient<NF, NSP, double, true>(s1, sU, u, sC, t, pJ, pdet, g);
+      mfmaGradient<NF, NSP, double>(s1, sU, u, sC, t, pJ, pdet, g);
     } else {
-      correctedGradient<D, P, NF, double, true>(s1, sU, sC, t, si, sj, sk, pJ, pdet, g);
+      correctedGradient<D, P, NF, double>(s1, sU, sC, t, si, sj, sk, pJ, pdet, g);
 #pragma unroll
       for (int d = 0; d < D; d++)
 #pragma unroll

@@ -394,7 +394,7 @@ __device__ __forceinline__ int mfmaFpt(int t, int r) {
 template <typename T>
 struct MfmaLane {
   T aD, aDT, aEzy, aEx;  // aDT: the transposed derivative matrix (FP64 layout)
-  int sx, sy, px, py, bx, by, ix, iy;
+  int px, py, bx, by, ix, iy;
   // FD: the derivative entries (aD, and the derivative rows of the FP32
   // operands) from the folded derivative OneD::DMF
   __device__ __forceinline__ MfmaLane(const T *s1, int t, bool FD = false) {
@@ -417,8 +417,8 @@ struct MfmaLane {
       aEx = m == 9 ? lL : m == 13 ? lR : d;
     }
     const int ln = t & 15, lp = t >> 4;
-    sx = lp + 4 * (ln & 3) + 16 * (ln >> 2);
-    sy = (ln & 3) + 4 * lp + 16 * (ln >> 2);
+    const int sx = lp + 4 * (ln & 3) + 16 * (ln >> 2);
+    const int sy = (ln & 3) + 4 * lp + 16 * (ln >> 2);
     px = padIdx<3>(sx);
     py = padIdx<3>(sy);
     bx = 4 * sx;
@@ -504,19 +504,19 @@ __device__ __forceinline__ void mfmaAxes(SM &sm, const int slot, const int t, co
   elementSync<64>();
 }
 
-// Face values of a state S held in LDS (one element, fields RS apart; padded
-// rows when PADV) at the lane's flux point of round r (mfmaFpt): round 0
+// Face values of a state S held in LDS (one element, fields RS apart, padded
+// rows) at the lane's flux point of round r (mfmaFpt): round 0
 // (faces 0-3) from the z lines -- the lane's own values own[] -- and the x
 // lines, round 1 (faces 4, 5) from the y lines.  All lanes take part.
-template <int NF, int RS, typename T, bool PADV = true>
+template <int NF, int RS, typename T>
 __device__ __forceinline__ void mfmaFaceRound(const T *s1, const T *S, const int t, const T (&own)[NF], const int r,
                                               T (&v)[NF]) {
   using V = MfmaVec<T>;
   const MfmaLane<T> L(s1, t);
-  const int ix = PADV ? L.px : L.sx, iy = PADV ? L.py : L.sy;
 #pragma unroll
   for (int k = 0; k < NF; k++)
-    v[k] = r == 0 ? V::ext(L.aEx, S[k * RS + ix], V::ext(L.aEzy, own[k], (T)0)) : V::ext(L.aEzy, S[k * RS + iy], (T)0);
+    v[k] = r == 0 ? V::ext(L.aEx, S[k * RS + L.px], V::ext(L.aEzy, own[k], (T)0))
+                  : V::ext(L.aEzy, S[k * RS + L.py], (T)0);
 }
 
 // mfmaFaceRound of values held only in registers (own[], one per lane): the
@@ -533,11 +533,11 @@ __device__ __forceinline__ void mfmaFaceRoundReg(const T *s1, const int t, const
 }
 
 // correctedGradient (below) for hex P3 with the reference-space derivative on
-// the matrix cores: the state S in LDS (fields RS apart, padded rows when
-// PADV) and the lane's own values own[], the jumps sCe [NF][NFP] at flux
+// the matrix cores: the state S in LDS (fields RS apart, padded
+// rows) and the lane's own values own[], the jumps sCe [NF][NFP] at flux
 // points numbered as fptLine numbers them.  Same terms; the matrix cores sum
 // the derivative's four products in their own order.  All lanes take part.
-template <int NF, int RS, typename T, bool PADV>
+template <int NF, int RS, typename T>
 __device__ __forceinline__ void mfmaGradient(const T *s1, const T *S, const T (&own)[NF], const T *sCe, const int t,
                                              const T *J, T detJ, T g[3][NF]) {
   using V = MfmaVec<T>;
@@ -554,7 +554,7 @@ __device__ __forceinline__ void mfmaGradient(const T *s1, const T *S, const T (&
   for (int d = 0; d < 3; d++) {
 #pragma unroll
     for (int k = 0; k < NF; k++) {
-      const T b = d == 2 ? own[k] : S[k * RS + (d == 0 ? (PADV ? L.px : L.sx) : (PADV ? L.py : L.sy))];
+      const T b = d == 2 ? own[k] : S[k * RS + (d == 0 ? L.px : L.py)];
       const T der = V::der(L.aD, d == 0 ? L.aEx : L.aEzy, b);
       const T dv = d < 2 ? lanePull(d == 0 ? L.ix : L.iy, der) : der;
       T corr = (T)0;
@@ -572,15 +572,14 @@ __device__ __forceinline__ void mfmaGradient(const T *s1, const T *S, const T (&
 // sum_m Dm u along each axis, plus correctU = correction * tNorm applied to the
 // flux-point jumps dUc (only the two faces normal to the axis are nonzero, in
 // ascending flux-point order), then transformed with JGinv / detJ.
-// sUe: [NF][NS] state, sCe: [NF][NFP] jumps, J: JGinv(dimRef, dimPhys).
-// PAD: sUe uses the padded LDS rows (ElemGeo::NSP, padIdx).
-template <int D, int P, int NF, typename T, bool PAD = false>
+// sUe: [NF][NSP] state (padded rows, padIdx), sCe: [NF][NFP] jumps, J:
+// JGinv(dimRef, dimPhys).
+template <int D, int P, int NF, typename T>
 __device__ __forceinline__ void correctedGradient(const T *s1, const T *sUe, const T *sCe, int t, int si, int sj,
                                                   int sk, const T *J, T detJ, T g[D][NF]) {
   using G = ElemGeo<D, P>;
   using O = OneD<P>;
-  constexpr int NFP = G::NFP, P1 = G::P1, NFACE = G::NFACE;
-  constexpr int NS = PAD ? G::NSP : G::NS;
+  constexpr int NSP = G::NSP, NFP = G::NFP, P1 = G::P1, NFACE = G::NFACE;
   int cq[NFACE], cside[NFACE], cax[NFACE];
   corrEntries<D, P>(t, cq, cside, cax);
   T cw[NFACE];  // lift weights, read once for all fields
@@ -596,7 +595,7 @@ __device__ __forceinline__ void correctedGradient(const T *s1, const T *sUe, con
 #pragma unroll
       for (int m = 0; m < P1; m++) {
         const int sp = (d == 0) ? m + P1 * (sj + P1 * sk) : (d == 1) ? si + P1 * (m + P1 * sk) : si + P1 * (sj + P1 * m);
-        acc += s1[O::DM + id * P1 + m] * sUe[k * NS + (PAD ? padIdx<P>(sp) : sp)];
+        acc += s1[O::DM + id * P1 + m] * sUe[k * NSP + padIdx<P>(sp)];
       }
       T corr = (T)0;
 #pragma unroll
@@ -919,9 +918,9 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
     if constexpr (VIS) {
       T g[D][NF], Fv[D][NF];
       if constexpr (MFF)
-        mfmaGradient<NF, G::NSP, T, true>(s1, &sU[slot][0][0], u, &sJ[slot][0][0], t, pJ, (T)pdet, g);
+        mfmaGradient<NF, G::NSP, T>(s1, &sU[slot][0][0], u, &sJ[slot][0][0], t, pJ, (T)pdet, g);
       else
-        correctedGradient<D, P, NF, T, true>(s1, &sU[slot][0][0], &sJ[slot][0][0], t, si, sj, sk, pJ, (T)pdet, g);
+        correctedGradient<D, P, NF, T>(s1, &sU[slot][0][0], &sJ[slot][0][0], t, si, sj, sk, pJ, (T)pdet, g);
       viscousFlux<D, NF, T>(a.ph, u, g, Fv);
 #pragma unroll
       for (int d = 0; d < D; d++)

@@ -419,10 +419,8 @@ __device__ __forceinline__ void boundaryState(const Phys &ph, int bc, const T *U
 // uses the physical tauxz = mu(du/dz + dw/dx), tauyz = mu(dv/dz + dw/dy),
 // Fv[0][3] = -tauxz.  Advection-diffusion: Fv = -diffD grad u
 // (viscousFluxAD, flux.cpp:361-366).
-// TG, the type of the gradient, may differ from T: the adjoint's state
-// passes differentiate through U only and keep the gradient in plain doubles.
-template <int D, int NF, typename T, typename TG = T>
-__device__ __forceinline__ void viscousFlux(const Phys &ph, const T *U, const TG g[D][NF], T Fv[D][NF]) {
+template <int D, int NF, typename T>
+__device__ __forceinline__ void viscousFlux(const Phys &ph, const T *U, const T g[D][NF], T Fv[D][NF]) {
   if constexpr (NF == 1) {
 #pragma unroll
     for (int d = 0; d < D; d++) Fv[d][0] = -(T)ph.diffD * g[d][0];
@@ -606,61 +604,6 @@ __device__ __forceinline__ void viscousShare(const Phys &ph, bool bnd, bool righ
     for (int d = 1; d < D; d++) acc += w[d] * F[d][NF - NV + k];
     C[k] = acc;
   }
-}
-
-// Adds the common LDG viscous normal flux sum_d Fc[d] n[d] to the inviscid
-// common flux Fn (face::calcViscousFlux, face.cpp:177-287), in the left
-// element's frame.  bnd: 0 interior, 1 Dirichlet-type boundary, 2 adiabatic
-// wall.
-template <int D, int NF, typename T, typename TG = T>
-__device__ __forceinline__ void ldgViscousFlux(const Phys &ph, int bnd, const T *UL, const T *UR, const TG gL[D][NF],
-                                               const TG gR[D][NF], const T *n, T *Fn) {
-  T Fc[D][NF];
-  if constexpr (NF == 1) {
-    // advection-diffusion: central flux of -diffD grad u (face.cpp:270-279)
-    T FL[D][NF], FR[D][NF];
-    viscousFlux<D, NF, T, TG>(ph, UL, gL, FL);
-    viscousFlux<D, NF, T, TG>(ph, UR, gR, FR);
-    T t = 0;
-#pragma unroll
-    for (int d = 0; d < D; d++) t += (T)0.5 * (FL[d][0] + FR[d][0]) * n[d];
-    Fn[0] += t;
-    return;
-  }
-  if (bnd) {
-    T Fb[D][NF];
-    if (bnd > 1) viscousFlux<D, NF, T, TG>(ph, UR, gR, Fb);
-    else viscousFlux<D, NF, T, TG>(ph, UL, gL, Fb);
-#pragma unroll
-    for (int d = 0; d < D; d++)
-#pragma unroll
-      for (int k = 0; k < NF; k++) Fc[d][k] = Fb[d][k] + (T)ph.tau * n[d] * (UL[k] - UR[k]);
-  } else {
-    T FL[D][NF], FR[D][NF];
-    viscousFlux<D, NF, T, TG>(ph, UL, gL, FL);
-    viscousFlux<D, NF, T, TG>(ph, UR, gR, FR);
-    const T pen = ldgPenalty<D, T>(ph, n);
-#pragma unroll
-    for (int k = 0; k < NF; k++) {
-      const T dF0 = FL[0][k] - FR[0][k], dF1 = FL[1][k] - FR[1][k];
-      const T dU = UL[k] - UR[k];
-      T nd;
-      if constexpr (D == 2) {
-        nd = n[0] * dF0 + n[1] * dF1;
-      } else {
-        // face.cpp:245 takes tempFL[1] here; viscFix = 1 takes tempFL[2]
-        const T dF2 = (ph.viscFix ? FL[2][k] : FL[1][k]) - FR[2][k];
-        nd = n[0] * dF0 + n[1] * dF1 + n[2] * dF2;
-      }
-#pragma unroll
-      for (int d = 0; d < D; d++)
-        Fc[d][k] = (T)0.5 * (FL[d][k] + FR[d][k]) + pen * n[d] * nd + (T)ph.tau * n[d] * dU;
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < NF; k++)
-#pragma unroll
-    for (int d = 0; d < D; d++) Fn[k] += Fc[d][k] * n[d];
 }
 
 }  // namespace frdev

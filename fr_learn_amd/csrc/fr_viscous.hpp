@@ -177,9 +177,9 @@ __global__ __launch_bounds__((ElemGeo<D, P>::NTH), 2) void k_visc_flux(StageArgs
   T g[D][NF];
   if (MG ? act : hasS) {
     if constexpr (MG) {
-      mfmaGradient<NF, NSP, T, true>(s1, &sU[slot][0][0], u, &sC[slot][0][0], t, pJ, pdet, g);
+      mfmaGradient<NF, NSP, T>(s1, &sU[slot][0][0], u, &sC[slot][0][0], t, pJ, pdet, g);
     } else {
-      correctedGradient<D, P, NF, T, true>(s1, &sU[slot][0][0], &sC[slot][0][0], t, si, sj, sk, pJ, pdet, g);
+      correctedGradient<D, P, NF, T>(s1, &sU[slot][0][0], &sC[slot][0][0], t, si, sj, sk, pJ, pdet, g);
 #pragma unroll
       for (int d = 0; d < D; d++)
 #pragma unroll
