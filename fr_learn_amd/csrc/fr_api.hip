@@ -129,7 +129,7 @@ frdev::StageArgs<T> makeStageArgs(fr_ctx *c, int in, int cur, int mode, int step
   a.divW = (T *)c->divF[step];  // completed in place, also where the update does not keep it
   // Inviscid quads and hexes store no intermediate stage state: a stage that
   // would read Us forms it from the base and the previous stage's residual
-  // (the viscous gradient kernel and the triangle kernels read Us itself).
+  // (k_visc_flux and the triangle kernels read Us itself).
   if (!c->cfg.viscous && !c->tri) {
     if (in == 1 && step > 0) {
       a.rprev = (const T *)c->divF[step - 1];
@@ -266,7 +266,7 @@ int usPoints(const fr_ctx *c, int NF) {
 
 // Small arrays go through pinned host memory that the layout kernels access
 // themselves: one buffer for the process, made and grown by the arrays that
-// pass it (a small solver's first one waits 10 us less than for 8 MB at once),
+// pass it (a small solver's first one waits 6 us less than for 8 MB at once),
 // freed with the last context.  A copy into the caller's pageable array costs
 // the runtime its pinning, most of all where the array is fresh, and a wait of
 // its own behind a busy stream: 74 KB 35 -> 6.5 us, 524 KB 60 -> 27 us, 40 arrays of
@@ -1121,8 +1121,8 @@ int fr_get_residual(fr_ctx *c, int step, double *out, int layout) {
 
 // Debug view of the residual's intermediate arrays (solver.hpp:55-61), for
 // the current state: one residual evaluation (as fr_calc_residual(ctx, 0))
-// with the stage kernel's (and on the viscous path the gradient kernel's)
-// debug outputs switched on, into buffers allocated for the call.
+// with the stage kernel's (and on the viscous path k_visc_flux's) debug outputs
+// switched on, into buffers allocated for the call.
 int fr_get_array(fr_ctx *c, int which, double *out) {
   if (!c || !out) return fail(FR_EINVAL, "null argument");
   if (which < 2 || which > 6) return fail(FR_EINVAL, "which: 2 F_spts, 3 Fn_fpts, 4 disFn_fpts, 5 dU_spts, 6 dU_fpts");

@@ -613,8 +613,10 @@ struct StageSmem {
   using G = ElemGeo<D, P, L>;
   // The contravariant fluxes of all axes are staged at once, so that the line
   // sums of every axis follow one synchronisation: one array per axis, the first
-  // later the updated state's.  Hexes, whose workgroups per CU the LDS would
-  // otherwise cost, put the last axis where the jump goes afterwards if it fits.
+  // later the updated state's.  Hexes P1, P2 and P4 put the last axis where the
+  // jump goes afterwards, which spares their workgroups per CU an array; P5's 216
+  // flux points do not hold its 252 padded rows, so it pays for two (49 KB a
+  // workgroup in FP64).
   // Hex P3 keeps them in registers (matrix cores).  These meshes wait on the
   // chain of LDS phases, not on bytes: with one synchronisation for two an axis,
   // P5 hexes (17 x 15 x 13, FP64, 200 steps of RK4) took 37.7 -> 35.4 ms, 40 mixed
@@ -1145,8 +1147,8 @@ __device__ __forceinline__ void stageBody(const StageArgs<T> &a, const int b, St
   // traces, so that sU keeps the stage state other elements of the block read.
   // (4) and (5) stand here and once more in the viscous update (viscUpdate):
   // called as one function, they came out with other code that took FP32 hex P3
-  // with the metrics formed in the kernel from 66 to 69 us a stage at 32^3 and
-  // from 224 to 234 at 48^3, whatever its arguments and register count.
+  // with the metrics formed in the kernel from 63 to 68 us a stage at 32^3 and
+  // from 216 to 231 at 48^3, whatever its arguments and register count.
   T utv[NF];  // the updated state at this thread's point, for the traces of (5)
   if (hasS) {
     int cq[NFACE], cside[NFACE], cax[NFACE];

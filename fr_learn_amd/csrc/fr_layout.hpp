@@ -42,11 +42,13 @@ constexpr int triTPEL(int P, int L) {
 }
 
 // Threads per element of a tensor-product element in tile layout L:
-// 0 (every per-mesh kernel): the solution-point count rounded up to a power of
-// two (at least 8), so that an element's threads never straddle a wavefront;
-// 1 (2D, a choice of the batched kernels' tuner): max(solution points, flux
-// points), packing e.g. seven P5 quads (36 points) into 252 threads where
-// layout 0 gives each 64 threads.
+// 0: the solution-point count rounded up to a power of two (at least 8), so
+// that an element's threads never straddle a wavefront;
+// 1 (2D): max(solution points, flux points), packing e.g. seven P5 quads (36
+// points) into 252 threads where layout 0 gives each 64 threads.
+// The per-mesh inviscid stage kernel takes layout 1 where stageTile says so (its
+// context's element blocks follow), the batched kernels where their tuner finds
+// it faster, every other kernel layout 0.
 constexpr int tensorTPE(int D, int P, int L) {
   const int P1 = P + 1, ns = (D == 3) ? P1 * P1 * P1 : P1 * P1, nf = (D == 3) ? 6 * P1 * P1 : 4 * P1;
   if (L == 1 && D == 2) return ns > nf ? ns : nf;
