@@ -8,6 +8,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <tuple>
 #include <type_traits>
 #include <utility>
 #include <vector>
@@ -313,6 +314,25 @@ double *stageBuffer(std::unique_lock<std::mutex> &lock, size_t bytes) {
   return gStage.buf;
 }
 
+// A launch by its own status: the thread's last error may be older and not ours,
+// and a read-back is not to fail for it.
+template <typename... P, typename... A>
+hipError_t launchRef(void (*k)(P...), unsigned blocks, int lds, hipStream_t st, A... args) {
+  std::tuple<P...> a(args...);
+  void *ptrs[sizeof...(P)];
+  int n = 0;
+  std::apply([&](auto &...x) { ((ptrs[n++] = (void *)&x), ...); }, a);
+  return hipLaunchKernel((const void *)k, dim3(blocks), dim3(256), ptrs, (size_t)lds, st);
+}
+// The end of a layout change: its stream is waited for whatever e is, since the
+// caller's array, the scratch and the pinned buffer are free for others after it.
+int refDone(fr_ctx *c, hipError_t e) {
+  const hipError_t w = hipStreamSynchronize(c->stream);
+  HIP_TRY(e);
+  HIP_TRY(w);
+  return 0;
+}
+
 int refToDev(fr_ctx *c, const double *src, double *dst, int NF, int NP) {
   const RefChunk r = refChunk(c, NF, NP, usPoints(c, NF));
   const size_t plane = (size_t)c->nE * NF;
@@ -320,21 +340,18 @@ int refToDev(fr_ctx *c, const double *src, double *dst, int NF, int NP) {
   if (double *buf = stageBuffer(lock, plane * NP * 8)) {
     const RefChunk w = refChunk(c, NF, NP, NP);
     std::memcpy(buf, src, plane * NP * 8);
-    hipLaunchKernelGGL(frdev::k_from_ref, dim3((c->nE + w.et - 1) / w.et), dim3(256), w.lds, c->stream, buf,
-                       c->ipermD, NF, NP, c->nE, w.et, 0, NP, dst);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return 0;
+    return refDone(c, launchRef(frdev::k_from_ref, nblk(c->nE, w.et), w.lds, c->stream, buf, c->ipermD, NF, NP, c->nE,
+                                w.et, 0, NP, dst));
   }
-  for (int p = 0; p < NP; p += r.pts) {
+  hipError_t e = hipSuccess;
+  for (int p = 0; p < NP && e == hipSuccess; p += r.pts) {
     const int np = std::min(r.pts, NP - p);
-    HIP_TRY(hipMemcpyAsync(c->Us, src + p * plane, np * plane * 8, hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(frdev::k_from_ref, dim3((c->nE + r.et - 1) / r.et), dim3(256), r.lds, c->stream,
-                       (const double *)c->Us, c->ipermD, NF, NP, c->nE, r.et, p, np, dst);
-    HIP_TRY(hipGetLastError());
+    e = hipMemcpyAsync(c->Us, src + p * plane, np * plane * 8, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess)
+      e = launchRef(frdev::k_from_ref, nblk(c->nE, r.et), r.lds, c->stream, (const double *)c->Us, c->ipermD, NF, NP,
+                    c->nE, r.et, p, np, dst);
   }
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  return 0;
+  return refDone(c, e);
 }
 template <bool ADD = false, typename TD>
 int devToRef(fr_ctx *c, const TD *src, double *dst, int NF, int NP, double add = 0.0) {
@@ -343,22 +360,21 @@ int devToRef(fr_ctx *c, const TD *src, double *dst, int NF, int NP, double add =
   std::unique_lock<std::mutex> lock(gStage.m, std::defer_lock);
   if (double *buf = stageBuffer(lock, plane * NP * 8)) {
     const RefChunk w = refChunk(c, NF, NP, NP);
-    hipLaunchKernelGGL((frdev::k_to_ref<TD, ADD>), dim3((c->nE + w.et - 1) / w.et), dim3(256), w.lds, c->stream, src,
-                       c->ipermD, NF, NP, c->nE, w.et, 0, NP, add, buf);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    const int rc = refDone(c, launchRef(frdev::k_to_ref<TD, ADD>, nblk(c->nE, w.et), w.lds, c->stream, src, c->ipermD, NF,
+                                        NP, c->nE, w.et, 0, NP, add, buf));
+    if (rc) return rc;
     std::memcpy(dst, buf, plane * NP * 8);
     return 0;
   }
-  for (int p = 0; p < NP; p += r.pts) {
+  hipError_t e = hipSuccess;
+  for (int p = 0; p < NP && e == hipSuccess; p += r.pts) {
     const int np = std::min(r.pts, NP - p);
-    hipLaunchKernelGGL((frdev::k_to_ref<TD, ADD>), dim3((c->nE + r.et - 1) / r.et), dim3(256), r.lds, c->stream, src,
-                       c->ipermD, NF, NP, c->nE, r.et, p, np, add, (double *)c->Us);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(dst + p * plane, c->Us, np * plane * 8, hipMemcpyDeviceToHost, c->stream));
+    e = launchRef(frdev::k_to_ref<TD, ADD>, nblk(c->nE, r.et), r.lds, c->stream, src, c->ipermD, NF, NP, c->nE, r.et, p,
+                  np, add, (double *)c->Us);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(dst + p * plane, c->Us, np * plane * 8, hipMemcpyDeviceToHost, c->stream);
   }
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  return 0;
+  return refDone(c, e);
 }
 
 int syncU32(fr_ctx *c) {
